@@ -74,7 +74,7 @@ struct Geo {
   static constexpr int kLdsBytes = kStages * kStageBytes;  // WQ8, WQ4 150,528; W1 147,456; W2 131,072
 };
 
-__device__ __forceinline__ int swz(int row) { return (row >> 2) & 3; }
+__device__ __forceinline__ int swz(int row) { return (row >> 1) & 3; }
 
 #define WIDE_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_f16((a), (b), (c), 0, 0, 0)
 
