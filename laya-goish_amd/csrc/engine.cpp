@@ -909,11 +909,13 @@ void Engine::run_layers_prefill(BatchPlan &b, lg_cancel_fn cancel, void *arg) {
   const int planes = split() ? 2 : 1;  // hi (+ lo) f16 planes per activation
   ws_x_.ensure(size_t(T) * d * 4);
   ws_h16_.ensure(size_t(T) * d * 2 * planes);
-  // q|k|v projections whose GEMM also rotates and stores q, k and v (the 256 x 256 exact GEMM's
-  // fused epilogue) leave no f32 q|k|v rows to stage
-  bool fused = split() && hd == 128;
+  // q|k|v projections whose GEMM also rotates and stores q, k and v (the exact GEMMs' fused epilogues) leave no f32
+  // q|k|v rows to stage
+  auto wide = [&](const ProjPart &p) { return hd == 128 && gemm_wide_takes(T, p.w, Epi::F32); };
+  bool fused = split();
   for (int l = 0; l < L && fused; ++l)
-    for (const ProjPart &p : layers_[l].qkv) fused = fused && p.col0 % 128 == 0 && gemm_wide_takes(T, p.w, Epi::F32);
+    for (const ProjPart &p : layers_[l].qkv)
+      fused = fused && p.col0 % hd == 0 && (wide(p) || gemm_mid_rope_takes(T, p.w, hd));
   if (!fused) ws_qkv_.ensure(size_t(T) * qkvw * 4);
   ws_q16_.ensure(size_t(T) * qw * 2 * planes);
   ws_att16_.ensure(size_t(T) * qw * 2 * planes);
@@ -951,25 +953,14 @@ void Engine::run_layers_prefill(BatchPlan &b, lg_cancel_fn cancel, void *arg) {
     ro.page_tokens = g.page_tokens;
     ro.qscale = attn_q_scale(hd);
     ro.kv_planes = kv_split() ? 2 : 1;
-    // short batches of F16 / Q8_0 weights: the small-tile q|k|v GEMM rotates and stores q, k and v too
-    // (no f32 q|k|v rows, no RoPE launch: C1's 144-token request 0.42 -> 0.40 ms, the same bits)
-    bool small_rope = split();
-    for (const ProjPart &p : ly.qkv) small_rope = small_rope && p.col0 % hd == 0 && gemm_small_rope_takes(T, p.w, hd);
     if (fused) {
       for (const ProjPart &p : ly.qkv) {
         ro.col0 = p.col0;
         const _Float16 *ks = chunk_sums(h16, h16lo, T, p.w);
         prof.begin_kernel("gemm");
-        if (!launch_gemm_wide_rope(h16, h16lo, T, p.w, p.bias, ro, stream, ks))
+        if (!wide(p)) launch_gemm_mid_rope(h16, h16lo, T, p.w, p.bias, ro, stream, ks);
+        else if (!launch_gemm_wide_rope(h16, h16lo, T, p.w, p.bias, ro, stream, ks))
           fail(LG_ERR_UNSUPPORTED, "gemm: fused q|k|v launch refused");
-        prof.end_kernel(double(p.w.bytes()) + double(T) * p.w.cols * 2, 2.0 * T * double(p.w.rows) * p.w.cols);
-      }
-    } else if (small_rope) {
-      for (const ProjPart &p : ly.qkv) {
-        ro.col0 = p.col0;
-        prof.begin_kernel("gemm");
-        if (!launch_gemm_small_rope(h16, h16lo, T, p.w, p.bias, ro, stream))
-          fail(LG_ERR_UNSUPPORTED, "gemm: short q|k|v launch refused");
         prof.end_kernel(double(p.w.bytes()) + double(T) * p.w.cols * 2, 2.0 * T * double(p.w.rows) * p.w.cols);
       }
     } else {

@@ -237,12 +237,16 @@ void Engine::run_laya(BatchPlan &b, const int32_t *qtype_dev, lg_cancel_fn cance
   prof.end(double(T) * d * 12, 0, stream);
   auto attention = [&](const LayaLayer &y, bool rope) {
     const float *cosT = y.full ? laya_cos_full_ : laya_cos_slide_, *sinT = y.full ? laya_sin_full_ : laya_sin_slide_;
-    // the 256 x 256 GEMM rotates q and k in its epilogue (the same bits as the RoPE kernel after it)
-    const bool fused = rope && x16lo && hd == 64 && (d / hd) % 2 == 0 && gemm_wide_takes(T, y.qkv.w, Epi::F32);
+    // the exact GEMMs rotate q and k in their epilogues (the same bits as the RoPE kernel after them)
+    const bool wide = rope && x16lo && hd == 64 && (d / hd) % 2 == 0 && gemm_wide_takes(T, y.qkv.w, Epi::F32);
+    const bool fused = wide || (rope && x16lo && hd == 64 && gemm_mid_laya_rope_takes(T, y.qkv.w));
     if (fused) {
       const _Float16 *ks = chunk_sums(x16, x16lo, T, y.qkv.w);
       prof.begin_kernel("gemm");
-      launch_gemm_wide_laya_rope(x16, x16lo, T, y.qkv.w, y.qkv.b, cosT, sinT, b.tok_pos, d / hd, qkv, 3 * d, stream, ks);
+      if (wide)
+        launch_gemm_wide_laya_rope(x16, x16lo, T, y.qkv.w, y.qkv.b, cosT, sinT, b.tok_pos, d / hd, qkv, 3 * d, stream, ks);
+      else
+        launch_gemm_mid_laya_rope(x16, x16lo, T, y.qkv.w, y.qkv.b, cosT, sinT, b.tok_pos, d / hd, qkv, 3 * d, stream);
       prof.end_kernel(double(y.qkv.w.bytes()) + double(T) * d * 2, 2.0 * T * double(y.qkv.w.rows) * d);
     } else {
       gemm(x16, x16lo, T, y.qkv.w, Epi::F32, qkv, nullptr, nullptr, 3 * d, y.qkv.b);

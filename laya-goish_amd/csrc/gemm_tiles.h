@@ -386,13 +386,253 @@ constexpr int lds_bytes() {
   return KIND == LG_Q4_K && MODE == SPLIT && corr > main ? corr : main;
 }
 
-// Epilogue of a q|k|v projection that rotates and stores q, k and v itself (RopeKvOut), as the RoPE
-// kernel would from the f32 rows: tiles of 64 weight rows (HN == 2), each wave's two 16-row blocks a
-// rotate-half pair of 16 dims each (d and d + hd/2 of one head), so the pair sits in one lane.
+// Epilogue of a q|k|v projection (gemm_mid.h) that rotates and stores q, k and v itself (RopeKvOut), as the RoPE
+// kernel would from the f32 rows: tiles of 64 weight rows (HN == 2), each wave's two 16-row blocks a rotate-half
+// pair of 16 dims each (d and d + hd/2 of one head), so the pair sits in one lane.  Row r of the launch is the row
+// ro_row0 + r of RopeKvOut's tables.
 constexpr int kTileEpiRope = 16;
+// The encoder's q|k|v projection: f32 rows as Epi::F32 stores them, q and k rotated (the same row map, head_dim 64).
+constexpr int kTileEpiLayaRope = 17;
+
+// Weight row of local weight-tile row r of tile nt (32 HN rows; 2 x 2 waves of 16 HN rows each).
+template <int EPI, int HN>
+__device__ __forceinline__ int tile_wrow(int r, int nt, int ffn, const RopeKvOut &ro) {
+  if (EPI == int(Epi::SWIGLU) || EPI == int(Epi::GEGLU)) {
+    // wave column r/(16 HN); 16-row block jb = (r/16) % HN: gate for jb < HN/2, up otherwise
+    const int wc = r / (16 * HN), jb = (r >> 4) % HN;
+    const int up = jb >= HN / 2, jj = jb % (HN / 2 > 0 ? HN / 2 : 1);
+    return up * ffn + nt * (16 * HN) + wc * (8 * HN) + jj * 16 + (r & 15);
+  }
+  if (EPI == kTileEpiRope || EPI == kTileEpiLayaRope) {
+    // tile nt: pair offsets 32 (nt % (hd/64)) .. + 32 of head nt / (hd/64) of this part; wave column
+    // r/32 takes 16 of them, block (r/16) % 2 the first or the second dim of each pair
+    const int hpt = ro.hd / 64, p = (nt % hpt) * 32 + (r / 32) * 16 + (r & 15);
+    return (nt / hpt) * ro.hd + p + ((r >> 4) & 1) * (ro.hd / 2);
+  }
+  return nt * (32 * HN) + r;
+}
+
+// Epilogue of a workgroup tile (32 HM) x (32 HN) of 2 x 2 waves, each (16 HM) x (16 HN): rows m0 .., column
+// tile nt, register r of acc[i][j] at row 16 i + 4 (lane / 16) + r, column 16 j + lane % 16 of the wave's part.
+template <int EPI, int HM, int HN>
+__device__ __forceinline__ void tile_epilogue(const f32x4 (&acc)[HM][HN], int M, int m0, int nt, int wm, int wn, int lane,
+                                              float *__restrict__ C, _Float16 *__restrict__ C16,
+                                              _Float16 *__restrict__ C16lo, int ldc, const float *__restrict__ bias,
+                                              const RopeKvOut &ro, int ro_row0) {
+  constexpr int MI = HM, NJ = HN, BNT = 32 * HN;
+  if constexpr (EPI == kTileEpiRope) {
+    // each lane holds dims d = p and d + hd/2 (blocks 0 and 1) of four rows; the values are the f32
+    // acc (+ bias) an F32 epilogue would store, rotated by rope_pair and split by split_f16 as the RoPE
+    // kernel does: q to scaled hi/lo planes [M][hq hd], k to its K page row, v to its V page column
+    const int hd = ro.hd, half = hd / 2, hpt = hd / 64;
+    const int p = (nt % hpt) * 32 + wn * 16 + (lane & 15);
+    const int pcol = (nt / hpt) * hd + p;  // output column of dim p within this part
+    const int head = (ro.col0 + pcol) / hd;
+    const int part = head < ro.hq ? 0 : head < ro.hq + ro.hkv ? 1 : 2;  // q, k, v
+    const int PT = ro.page_tokens, plane = PT * hd, kvp = ro.kv_planes;
+    const float b0 = bias ? bias[pcol] : 0.0f, b1 = bias ? bias[pcol + half] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      // the block's four rows: positions and pages, then every table value, in one round trip each (rows past
+      // M read row M - 1 and are not stored)
+      const int rb = m0 + wm * (16 * HM) + i * 16 + (lane >> 4) * 4;
+      int pos[4], page[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int grow = ro_row0 + min(rb + r, M - 1);
+        pos[r] = ro.tok_pos[grow];
+        page[r] = ro.tok_page[grow];
+      }
+      float v0[4], v1[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v0[r] = acc[i][0][r];
+        v1[r] = acc[i][1][r];
+        if (bias) {
+          v0[r] += b0;
+          v1[r] += b1;
+        }
+      }
+      if (part < 2) {
+        float cs[4][4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int64_t tb = int64_t(pos[r]) * hd + p;
+          cs[r][0] = ro.cosT[tb];
+          cs[r][1] = ro.sinT[tb];
+          cs[r][2] = ro.cosT[tb + half];
+          cs[r][3] = ro.sinT[tb + half];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (rb + r >= M) continue;
+          const int grow = ro_row0 + rb + r;
+          _Float16 h, l;
+          float a, c;
+          rope_pair(v0[r], v1[r], cs[r][0], cs[r][1], cs[r][2], cs[r][3], a, c);
+          if (part == 0) {
+            _Float16 *dh = ro.q16 + int64_t(grow) * (ro.hq * hd) + head * hd + p;
+            _Float16 *dl = ro.q16lo + int64_t(grow) * (ro.hq * hd) + head * hd + p;
+            split_f16(a * ro.qscale, h, l);
+            dh[0] = h;
+            dl[0] = l;
+            split_f16(c * ro.qscale, h, l);
+            dh[half] = h;
+            dl[half] = l;
+          } else {
+            const int64_t blk = int64_t(page[r]) * ro.page_stride + int64_t(head - ro.hq) * plane;
+            _Float16 *dh = ro.kpool + kvp * blk + (pos[r] % PT) * hd + p;
+            split_f16(a, h, l);
+            dh[0] = h;
+            if (kvp == 2) dh[plane] = l;
+            split_f16(c, h, l);
+            dh[half] = h;
+            if (kvp == 2) dh[plane + half] = l;
+          }
+        }
+      } else {
+        // V page columns: four rows that are consecutive positions of one page from a multiple of 4 take one
+        // 8-byte store a column and plane, others one slot at a time
+        typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+        bool quad = rb + 3 < M && (pos[0] & 3) == 0 && (PT & 3) == 0;
+#pragma unroll
+        for (int r = 1; r < 4; ++r) quad = quad && pos[r] == pos[0] + r && page[r] == page[0];
+        half4 h0, l0, h1, l1;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          _Float16 h, l;
+          split_f16(v0[r], h, l);
+          h0[r] = h;
+          l0[r] = l;
+          split_f16(v1[r], h, l);
+          h1[r] = h;
+          l1[r] = l;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (rb + r >= M) continue;
+          const int64_t blk = int64_t(page[r]) * ro.page_stride + int64_t(head - ro.hq - ro.hkv) * plane;
+          _Float16 *d0 = ro.vpool + kvp * blk + int64_t(p) * PT + (pos[r] % PT), *d1 = d0 + int64_t(half) * PT;
+          if (quad) {
+            *reinterpret_cast<half4 *>(d0) = h0;
+            *reinterpret_cast<half4 *>(d1) = h1;
+            if (kvp == 2) {
+              *reinterpret_cast<half4 *>(d0 + plane) = l0;
+              *reinterpret_cast<half4 *>(d1 + plane) = l1;
+            }
+            break;
+          }
+          d0[0] = h0[r];
+          d1[0] = h1[r];
+          if (kvp == 2) {
+            d0[plane] = l0[r];
+            d1[plane] = l1[r];
+          }
+        }
+      }
+    }
+    return;
+  }
+
+  if constexpr (EPI == kTileEpiLayaRope) {
+    // one 64-dim head of q, k or v: each lane holds dims p and p + 32 of four rows, q and k rotated by rope_pair
+    // as the encoder's RoPE kernel rotates the F32 epilogue's values
+    const int p = wn * 16 + (lane & 15), col = nt * 64 + p;
+    const bool rot = nt < 2 * ro.hq;
+    const float b0 = bias ? bias[col] : 0.0f, b1 = bias ? bias[col + 32] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const int rb = m0 + wm * (16 * HM) + i * 16 + (lane >> 4) * 4;
+      float cs[4][4] = {};
+      if (rot) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int64_t tb = int64_t(ro.tok_pos[ro_row0 + min(rb + r, M - 1)]) * 64 + p;
+          cs[r][0] = ro.cosT[tb];
+          cs[r][1] = ro.sinT[tb];
+          cs[r][2] = ro.cosT[tb + 32];
+          cs[r][3] = ro.sinT[tb + 32];
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (rb + r >= M) continue;
+        float v0 = acc[i][0][r], v1 = acc[i][1][r];
+        if (bias) {
+          v0 += b0;
+          v1 += b1;
+        }
+        if (rot) {
+          float a, c;
+          rope_pair(v0, v1, cs[r][0], cs[r][1], cs[r][2], cs[r][3], a, c);
+          v0 = a;
+          v1 = c;
+        }
+        C[int64_t(rb + r) * ldc + col] = v0;
+        C[int64_t(rb + r) * ldc + col + 32] = v1;
+      }
+    }
+    return;
+  }
+
+  // epilogue: acc[i][j] register r -> row 16 i + 4 (lane / 16) + r, column 16 j + lane % 16 of the
+  // wave tile
+  const int col_in = lane & 15;
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    // the residual add reads a 16-row block's values first, all in one round trip (rows past M read
+    // row M - 1 and are not stored)
+    float cv[4][EPI == int(Epi::ADD) ? NJ : 1];
+    if constexpr (EPI == int(Epi::ADD)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = min(m0 + wm * (16 * HM) + i * 16 + (lane >> 4) * 4 + r, M - 1);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) cv[r][j] = C[int64_t(row) * ldc + nt * BNT + wn * (16 * HN) + j * 16 + col_in];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = m0 + wm * (16 * HM) + i * 16 + (lane >> 4) * 4 + r;
+      if (row >= M) continue;
+      if (EPI == int(Epi::SWIGLU) || EPI == int(Epi::GEGLU)) {
+        // gate block j pairs with up block j + NJ / 2 (the same output columns)
+#pragma unroll
+        for (int j = 0; j < NJ / 2; ++j) {
+          const int col = nt * (BNT / 2) + wn * (8 * HN) + j * 16 + col_in;
+          const float g = acc[i][j][r];
+          const float v = (EPI == int(Epi::SWIGLU) ? silu(g) : gelu_tanh(g)) * acc[i][j + NJ / 2][r];
+          _Float16 h, hl;
+          split_f16(v, h, hl);
+          C16[int64_t(row) * ldc + col] = h;
+          if (C16lo) C16lo[int64_t(row) * ldc + col] = hl;
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const int col = nt * BNT + wn * (16 * HN) + j * 16 + col_in;
+          float v = acc[i][j][r];
+          if (EPI == int(Epi::F32)) {
+            if (bias) v += bias[col];
+            C[int64_t(row) * ldc + col] = v;
+          } else if constexpr (EPI == int(Epi::ADD)) {
+            if (bias) v += bias[col];
+            C[int64_t(row) * ldc + col] = cv[r][j] + v;
+          } else {
+            if (bias) v += bias[col];
+            if (EPI == int(Epi::RELU16)) v = fmaxf(v, 0.0f);
+            _Float16 h, hl;
+            split_f16(v, h, hl);
+            C16[int64_t(row) * ldc + col] = h;
+            if (C16lo) C16lo[int64_t(row) * ldc + col] = hl;
+          }
+        }
+      }
+    }
+  }
+}
 
 // ks / kslo: the chunk-sum planes of a two-pass Q4_K launch ([M][W.pkp] each), unused otherwise.
-// ro: the q|k|v outputs of EPI == kTileEpiRope (row r of the launch is ro's row ro_row0 + r).
 template <uint32_t KIND, int EPI, int MODE, int BK, int HM, int HN, int STAGES>
 __global__ __launch_bounds__(256) void gemm_kernel(const _Float16 *__restrict__ A,
                                                    const _Float16 *__restrict__ Alo, int M, int K,
@@ -401,14 +641,13 @@ __global__ __launch_bounds__(256) void gemm_kernel(const _Float16 *__restrict__ 
                                                    _Float16 *__restrict__ C16lo, int ldc,
                                                    const float *__restrict__ bias, int MT, int NT,
                                                    int ffn, const _Float16 *__restrict__ ks,
-                                                   const _Float16 *__restrict__ kslo, RopeKvOut ro, int ro_row0) {
+                                                   const _Float16 *__restrict__ kslo) {
   using CF = Cfg<MODE, BK, HM, HN, STAGES>;
   constexpr int BMW = CF::kBM, BNT = CF::kBN, LDK = CF::kLDK;
   constexpr bool kSplitA = CF::kSplitA, kSplitB = CF::kSplitB;
   constexpr bool kScaled = MODE == SPLIT && (KIND == LG_Q8_0 || KIND == LG_Q4_K);
   static_assert(HN % 2 == 0 || (EPI != int(Epi::SWIGLU) && EPI != int(Epi::GEGLU)),
                 "gated epilogues pair gate and up blocks inside a wave");
-  static_assert(EPI != kTileEpiRope || HN == 2, "the rotating epilogue takes 64-row tiles");
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -424,22 +663,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(const _Float16 *__restrict__ 
     Bl = kSplitB ? Bs + CF::kBPlane : Bs;
     Ds = reinterpret_cast<float *>(base + CF::kStageHalves);
   };
-  // local weight-tile row -> weight row
-  auto wrow = [&](int r) -> int {
-    if (EPI == int(Epi::SWIGLU) || EPI == int(Epi::GEGLU)) {
-      // wave column r/(16 HN); 16-row block jb = (r/16) % HN: gate for jb < HN/2, up otherwise
-      const int wc = r / (16 * HN), jb = (r >> 4) % HN;
-      const int up = jb >= HN / 2, jj = jb % (HN / 2);
-      return up * ffn + nt * (BNT / 2) + wc * (8 * HN) + jj * 16 + (r & 15);
-    }
-    if (EPI == kTileEpiRope) {
-      // tile nt: pair offsets 32 (nt % (hd/64)) .. + 32 of head nt / (hd/64) of this part; wave column
-      // r/32 takes 16 of them, block (r/16) % 2 the first or the second dim of each pair
-      const int hpt = ro.hd / 64, p = (nt % hpt) * 32 + (r / 32) * 16 + (r & 15);
-      return (nt / hpt) * ro.hd + p + ((r >> 4) & 1) * (ro.hd / 2);
-    }
-    return nt * BNT + r;
-  };
+  auto wrow = [&](int r) -> int { return tile_wrow<EPI, HN>(r, nt, ffn, RopeKvOut{}); };
 
   using BL = BLoad<KIND, MODE, BK, BNT>;
   using AL = ALoad<BMW, BK, kSplitA>;
@@ -547,125 +771,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(const _Float16 *__restrict__ 
     }
   }
 
-  if constexpr (EPI == kTileEpiRope) {
-    // each lane holds dims d = p and d + hd/2 (blocks 0 and 1) of four rows; the values are the f32
-    // acc (+ bias) an F32 epilogue would store, rotated by rope_pair and split by split_f16 as the RoPE
-    // kernel does: q to scaled hi/lo planes [M][hq hd], k to its K page row, v to its V page column
-    const int hd = ro.hd, half = hd / 2, hpt = hd / 64;
-    const int p = (nt % hpt) * 32 + wn * 16 + (lane & 15);
-    const int pcol = (nt / hpt) * hd + p;  // output column of dim p within this part
-    const int head = (ro.col0 + pcol) / hd;
-    const int part = head < ro.hq ? 0 : head < ro.hq + ro.hkv ? 1 : 2;  // q, k, v
-    const int PT = ro.page_tokens, plane = PT * hd, kvp = ro.kv_planes;
-    const float b0 = bias ? bias[pcol] : 0.0f, b1 = bias ? bias[pcol + half] : 0.0f;
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm * (16 * HM) + i * 16 + (lane >> 4) * 4 + r;
-        if (row >= M) continue;
-        const int grow = ro_row0 + row;
-        const int pos = ro.tok_pos[grow];
-        const int64_t page = ro.tok_page[grow];
-        float v0 = acc[i][0][r], v1 = acc[i][1][r];
-        if (bias) {
-          v0 += b0;
-          v1 += b1;
-        }
-        _Float16 h, l;
-        if (part < 2) {
-          const int64_t tb = int64_t(pos) * hd + p;
-          float a, c;
-          rope_pair(v0, v1, ro.cosT[tb], ro.sinT[tb], ro.cosT[tb + half], ro.sinT[tb + half], a, c);
-          if (part == 0) {
-            _Float16 *dh = ro.q16 + int64_t(grow) * (ro.hq * hd) + head * hd + p;
-            _Float16 *dl = ro.q16lo + int64_t(grow) * (ro.hq * hd) + head * hd + p;
-            split_f16(a * ro.qscale, h, l);
-            dh[0] = h;
-            dl[0] = l;
-            split_f16(c * ro.qscale, h, l);
-            dh[half] = h;
-            dl[half] = l;
-          } else {
-            const int64_t blk = page * ro.page_stride + int64_t(head - ro.hq) * plane;
-            _Float16 *dh = ro.kpool + kvp * blk + (pos % PT) * hd + p;
-            split_f16(a, h, l);
-            dh[0] = h;
-            if (kvp == 2) dh[plane] = l;
-            split_f16(c, h, l);
-            dh[half] = h;
-            if (kvp == 2) dh[plane + half] = l;
-          }
-        } else {
-          const int64_t blk = page * ro.page_stride + int64_t(head - ro.hq - ro.hkv) * plane;
-          _Float16 *dh = ro.vpool + kvp * blk + int64_t(p) * PT + (pos % PT);
-          split_f16(v0, h, l);
-          dh[0] = h;
-          if (kvp == 2) dh[plane] = l;
-          split_f16(v1, h, l);
-          dh[int64_t(half) * PT] = h;
-          if (kvp == 2) dh[plane + int64_t(half) * PT] = l;
-        }
-      }
-    }
-    return;
-  }
-
-  // epilogue: acc[i][j] register r -> row 16 i + 4 (lane / 16) + r, column 16 j + lane % 16 of the
-  // wave tile
-  const int col_in = lane & 15;
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    // the residual add reads a 16-row block's values first, all in one round trip (rows past M read
-    // row M - 1 and are not stored)
-    float cv[4][EPI == int(Epi::ADD) ? NJ : 1];
-    if constexpr (EPI == int(Epi::ADD)) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = min(m0 + wm * (16 * HM) + i * 16 + (lane >> 4) * 4 + r, M - 1);
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) cv[r][j] = C[int64_t(row) * ldc + nt * BNT + wn * (16 * HN) + j * 16 + col_in];
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = m0 + wm * (16 * HM) + i * 16 + (lane >> 4) * 4 + r;
-      if (row >= M) continue;
-      if (EPI == int(Epi::SWIGLU) || EPI == int(Epi::GEGLU)) {
-        // gate block j pairs with up block j + NJ / 2 (the same output columns)
-#pragma unroll
-        for (int j = 0; j < NJ / 2; ++j) {
-          const int col = nt * (BNT / 2) + wn * (8 * HN) + j * 16 + col_in;
-          const float g = acc[i][j][r];
-          const float v = (EPI == int(Epi::SWIGLU) ? silu(g) : gelu_tanh(g)) * acc[i][j + NJ / 2][r];
-          _Float16 h, hl;
-          split_f16(v, h, hl);
-          C16[int64_t(row) * ldc + col] = h;
-          if (C16lo) C16lo[int64_t(row) * ldc + col] = hl;
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          const int col = nt * BNT + wn * (16 * HN) + j * 16 + col_in;
-          float v = acc[i][j][r];
-          if (EPI == int(Epi::F32)) {
-            if (bias) v += bias[col];
-            C[int64_t(row) * ldc + col] = v;
-          } else if constexpr (EPI == int(Epi::ADD)) {
-            if (bias) v += bias[col];
-            C[int64_t(row) * ldc + col] = cv[r][j] + v;
-          } else {
-            if (bias) v += bias[col];
-            if (EPI == int(Epi::RELU16)) v = fmaxf(v, 0.0f);
-            _Float16 h, hl;
-            split_f16(v, h, hl);
-            C16[int64_t(row) * ldc + col] = h;
-            if (C16lo) C16lo[int64_t(row) * ldc + col] = hl;
-          }
-        }
-      }
-    }
-  }
+  tile_epilogue<EPI, HM, HN>(acc, M, m0, nt, wm, wn, lane, C, C16, C16lo, ldc, bias, RopeKvOut{}, 0);
 }
 
 template <uint32_t KIND, int MODE, int BK, int HM, int HN, int STAGES>
@@ -708,7 +814,7 @@ bool launch_cfg(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &
     auto fn = gemm_kernel<KIND, E, MODE, BK, HM, HN, STAGES>;                                                  \
     grant_lds(reinterpret_cast<const void *>(fn), lds);                                                        \
     launch_timed(fn, grid, block, lds, st, Ac, Alc, Mc, K, W, Cc, C16c, C16lc, ldc, bias, MT, NT, ffn, ksc,     \
-                 kslc, RopeKvOut{}, 0);                                                                        \
+                 kslc);                                                                                        \
   } while (0)
     switch (epi) {
       case Epi::F32: LAUNCH(0); break;
@@ -729,27 +835,6 @@ bool launch_cfg(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &
   return true;
 }
 
-// The q|k|v projection (or a column range of it, ro.col0 a multiple of hd) on tiles of BM x 64 weight
-// rows with the rotating epilogue; false (nothing launched) when the shape does not fit.
-template <uint32_t KIND, int MODE, int BK, int HM, int STAGES>
-bool launch_cfg_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, const float *bias,
-                     const RopeKvOut &ro, hipStream_t st, const _Float16 *ks = nullptr) {
-  using CF = Cfg<MODE, BK, HM, 2, STAGES>;
-  if ((ro.hd != 64 && ro.hd != 128) || W.rows % ro.hd || ro.col0 % ro.hd || !Alo || !ro.q16lo) return false;
-  const int K = W.cols, NT = W.rows / 64;
-  const int64_t rows_cap = ((1ll << 31) - 1) / (int64_t(K) * 2) / CF::kBM * CF::kBM;
-  if (int64_t(M) > rows_cap) return false;
-  const int MT = (M + CF::kBM - 1) / CF::kBM;
-  const dim3 grid(MT * NT), block(256);
-  constexpr int lds = lds_bytes<KIND, MODE, BK, HM, 2, STAGES>();
-  auto fn = gemm_kernel<KIND, kTileEpiRope, MODE, BK, HM, 2, STAGES>;
-  grant_lds(reinterpret_cast<const void *>(fn), lds);
-  const _Float16 *kslc = ks ? ks + int64_t(M) * W.pkp : nullptr;
-  launch_timed(fn, grid, block, lds, st, A, Alo, M, K, W, static_cast<float *>(nullptr), static_cast<_Float16 *>(nullptr),
-               static_cast<_Float16 *>(nullptr), 0, bias, MT, NT, W.rows / 2, ks, kslc, ro, 0);
-  return true;
-}
-
 }  // namespace
 
 // Exact Q8_0 tiles, built in their own translation unit (k_gemm_q8.hip) with MFMA results in
@@ -757,9 +842,6 @@ bool launch_cfg_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMat
 bool launch_gemm_q8_exact(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi,
                           float *C, _Float16 *C16, _Float16 *C16lo, int ldc, const float *bias,
                           hipStream_t st);
-// launch_gemm_small_rope for Q8_0 weights (the exact Q8_0 tiles' translation unit).
-bool launch_gemm_q8_small_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, const float *bias,
-                               const RopeKvOut &ro, hipStream_t st);
 // Exact two-pass Q4_K tiles (the same translation unit): codes, sub-block scales and the correction
 // over the activation's chunk sums ks.
 bool launch_gemm_q4_exact(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi,
@@ -774,5 +856,12 @@ bool launch_gemm_q4_exact(const _Float16 *A, const _Float16 *Alo, int M, const D
 bool launch_gemm_wide(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi, float *C,
                       _Float16 *C16, _Float16 *C16lo, int ldc, const float *bias, hipStream_t st,
                       const _Float16 *ks = nullptr);
+
+// Exact GEMM over the weight's prefill copy on the tiles of gemm_mid.h, for what launch_gemm_wide leaves: any M, the
+// same bits.  Returns false (nothing launched) when the matrix has no prefill copy or the shape or epilogue is not
+// one it takes.
+bool launch_gemm_mid(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi, float *C,
+                     _Float16 *C16, _Float16 *C16lo, int ldc, const float *bias, hipStream_t st,
+                     const _Float16 *ks = nullptr);
 
 }  // namespace lg

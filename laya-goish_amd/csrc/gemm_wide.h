@@ -48,6 +48,20 @@ constexpr int kEpiRopeKv = 16;
 // (head_dim 64; RopeKvOut's cosT, sinT, tok_pos and hq)
 constexpr int kEpiLayaRope = 17;
 
+// The mode of W's prefill copy, or -1 when it has none.
+inline int prefill_mode(const DevMatrix &W) {
+  if (!W.pc) return -1;
+  switch (W.kind) {
+    case LG_Q8_0: return W.pcs ? WQ8 : -1;
+    case LG_F16: return W1;
+    case LG_Q4_K:  // the two-pass copy (codes, scales, correction planes), or hi/lo planes
+      if (needs_ksum(W)) return W.pcs && W.pcl ? WQ4 : -1;
+      return W.pcl ? W2 : -1;
+    case LG_Q6_K: return W.pcl ? W2 : -1;
+    default: return -1;
+  }
+}
+
 constexpr int BM = 256, BN = 256, BK = 32, WAVES = 8, THREADS = 64 * WAVES;
 constexpr int ROWB = BK * 2;      // bytes per LDS row of one plane
 constexpr int PLANE = BM * ROWB;  // 16 KiB

@@ -1,0 +1,228 @@
+// Launches of the exact GEMM tiles of gemm_mid.h, and the choice between them and the 256 x 256 tiles.  Built with
+// MFMA results in VGPRs (-mllvm -amdgpu-mfma-vgpr-form), as k_gemm_q8.hip.
+#include <algorithm>
+
+#include "gemm_mid.h"
+
+namespace lg {
+namespace {
+
+using wide::W1;
+using wide::W2;
+using wide::WQ4;
+using wide::WQ8;
+
+// Tile configurations: (HM, HN, stages).
+enum Tile { T11, T12, T22, T24, T24D, T44, kTiles, kNoTile = -1 };
+
+// Microseconds per 64-deep K step of one workgroup alone on a CU (one) and of two sharing it (two): (launch time -
+// 3 us) / (K / 64) over M 24-1437 and the q|k|v, o, gate|up and down shapes of the workload models (weights rotating
+// through 1.4 GB).  Two where the LDS holds a single workgroup is twice one.  0: not a configuration of the mode.
+struct StepCost {
+  float one, two;
+};
+constexpr StepCost kCost[4][kTiles] = {
+    /* WQ8 */ {{0.24f, 0.40f}, {0.31f, 0.54f}, {0.46f, 0.78f}, {0.84f, 1.03f}, {0.70f, 1.40f}, {1.11f, 2.25f}},
+    /* W1  */ {{0.20f, 0.36f}, {0.24f, 0.47f}, {0.36f, 0.70f}, {0.80f, 0.92f}, {0.57f, 1.14f}, {0.95f, 1.90f}},
+    /* W2  */ {{0.27f, 0.50f}, {0.43f, 0.86f}, {0.49f, 0.98f}, {0, 0}, {0.85f, 1.70f}, {1.50f, 3.00f}},
+    /* WQ4 */ {{0.24f, 0.40f}, {0.31f, 0.54f}, {0.46f, 0.78f}, {0, 0}, {0.70f, 1.40f}, {1.11f, 2.25f}},
+};
+constexpr int kHM[kTiles] = {1, 1, 2, 2, 2, 4}, kHN[kTiles] = {1, 2, 2, 4, 4, 4};
+// a 256 x 256 tile's microseconds per 64-deep step, one workgroup per CU (mode order as above)
+constexpr float kWideStep[4] = {3.6f, 3.0f, 4.9f, 3.6f};
+
+int cus() { return device_cus(); }
+
+// Rounds of two workgroups per CU, the last one alone when half a round or less is left.
+float cost(const StepCost &c, int64_t tiles) {
+  const int64_t n = cus(), rounds = tiles / (2 * n), rest = tiles - rounds * 2 * n;
+  return float(rounds) * c.two + (rest == 0 ? 0.0f : rest <= n ? c.one : c.two);
+}
+
+// The cheapest configuration for M rows of a matrix of `rows` weight rows (only those of 64 columns when rope), and
+// its cost; kNoTile when none divides the output.
+int best_tile(int mode, int M, int rows, bool glu, bool rope, float *best) {
+  int t = kNoTile;
+  for (int i = 0; i < kTiles; ++i) {
+    const int bm = 32 * kHM[i], bn = 32 * kHN[i];
+    if (kCost[mode][i].one == 0 || rows % bn || (glu && kHN[i] % 2) || (rope && kHN[i] != 2)) continue;
+    const float c = cost(kCost[mode][i], int64_t((M + bm - 1) / bm) * (rows / bn));
+    if (t == kNoTile || c < *best) {
+      t = i;
+      *best = c;
+    }
+  }
+  return t;
+}
+
+// the mode of an M-row launch of W, or -1 when these tiles do not take it
+int mid_mode(int M, const DevMatrix &W) {
+  const int mode = wide::prefill_mode(W);
+  if (M <= 0 || mode < 0 || W.cols % mid::BK != 0) return -1;
+  if (int64_t(W.rows) * W.cols * 2 >= (int64_t(1) << 32)) return -1;  // 32-bit buffer offsets of the weights
+  return mode;
+}
+
+struct Launch {
+  const _Float16 *A, *Alo;
+  int M;
+  const DevMatrix &W;
+  float *C;
+  _Float16 *C16, *C16lo;
+  int ldc;
+  const float *bias;
+  const RopeKvOut &ro;
+  hipStream_t st;
+  const _Float16 *ks;
+};
+
+template <int EPI, int MODE, int HM, int HN, int S>
+void launch_rows(const Launch &l) {
+  const DevMatrix &W = l.W;
+  const int N = W.rows, K = W.cols, NT = N / (32 * HN);
+  constexpr int BM = 32 * HM, lds = mid::lds_bytes<MODE, HM, HN, S>();
+  // activation rows per launch: the planes' buffer offsets are 32-bit
+  const int64_t rows_cap = ((int64_t(1) << 31) - 1) / (int64_t(K) * 2) / BM * BM;
+  LG_REQUIRE(rows_cap > 0, "gemm: K=%d too large", K);
+  const auto fn = mid::gemm_mid_kernel<EPI, MODE, HM, HN, S>;
+  grant_lds(reinterpret_cast<const void *>(fn), lds);
+  KernelTimer *timer = kernel_timer();
+  const KernelTimer whole = timer ? *timer : KernelTimer{};
+  for (int m0 = 0; m0 < l.M;) {
+    const int Mc = int(std::min<int64_t>(l.M - m0, rows_cap));
+    if (timer) {
+      timer->start = m0 == 0 ? whole.start : nullptr;
+      timer->stop = m0 + Mc >= l.M ? whole.stop : nullptr;
+    }
+    const int MT = (Mc + BM - 1) / BM;
+    LG_REQUIRE(int64_t(MT) * NT < (int64_t(1) << 31), "gemm: grid too large");
+    wide::KqCorr kq;
+    if (MODE == WQ4) {
+      kq.kp = W.pkp;
+      kq.ks = l.ks + int64_t(m0) * W.pkp;
+      kq.kslo = l.ks + (int64_t(l.M) + m0) * W.pkp;
+      kq.bh = W.pcl;
+      kq.bl = W.pcl + int64_t(N) * W.pkp;
+      kq.rs = W.pcr;
+    }
+    const int64_t co = int64_t(m0) * l.ldc;
+    launch_timed(fn, dim3(MT * NT), dim3(256), lds, l.st, l.A + int64_t(m0) * K, l.Alo + int64_t(m0) * K, Mc, K,
+                 static_cast<const _Float16 *>(W.pc), static_cast<const _Float16 *>(W.pcl),
+                 static_cast<const float *>(W.pcs), N, l.C ? l.C + co : nullptr, l.C16 ? l.C16 + co : nullptr,
+                 l.C16lo ? l.C16lo + co : nullptr, l.ldc, l.bias, MT, NT, N / 2, l.ro, m0, kq);
+    m0 += Mc;
+  }
+  if (timer) *timer = whole;
+  HIP_CHECK(hipGetLastError());
+}
+
+template <int EPI, int MODE>
+void launch_tile(int tile, const Launch &l) {
+  constexpr bool kRope = EPI == kTileEpiRope || EPI == kTileEpiLayaRope;
+  constexpr bool kGlu = EPI == int(Epi::SWIGLU) || EPI == int(Epi::GEGLU);
+  constexpr bool w2 = MODE == W2, wq4 = MODE == WQ4;
+  switch (tile) {
+    case T11:
+      if constexpr (!kRope && !kGlu) launch_rows<EPI, MODE, 1, 1, w2 ? 5 : 6>(l);
+      break;
+    case T12: launch_rows<EPI, MODE, 1, 2, w2 ? 3 : 4>(l); break;
+    case T22: launch_rows<EPI, MODE, 2, 2, w2 ? 4 : 3>(l); break;
+    case T24:  // two workgroups per CU
+      if constexpr (!kRope && !w2 && !wq4) launch_rows<EPI, MODE, 2, 4, 2>(l);
+      break;
+    case T24D:  // one, with more steps in flight
+      if constexpr (!kRope) launch_rows<EPI, MODE, 2, 4, w2 ? 3 : 4>(l);
+      break;
+    case T44:
+      if constexpr (!kRope) launch_rows<EPI, MODE, 4, 4, 2>(l);
+      break;
+  }
+}
+
+template <int EPI>
+void launch_mode(int mode, int tile, const Launch &l) {
+  // GeGLU, ReLU and the encoder's rotation come with F16 weights only
+  constexpr bool kF16Only = EPI == int(Epi::GEGLU) || EPI == int(Epi::RELU16) || EPI == kTileEpiLayaRope;
+  if constexpr (kF16Only) {
+    launch_tile<EPI, W1>(tile, l);
+  } else {
+    if (mode == WQ8) launch_tile<EPI, WQ8>(tile, l);
+    else if (mode == W1) launch_tile<EPI, W1>(tile, l);
+    else if (mode == W2) launch_tile<EPI, W2>(tile, l);
+    else launch_tile<EPI, WQ4>(tile, l);
+  }
+}
+
+}  // namespace
+
+bool gemm_mid_ahead(int M, const DevMatrix &W, bool glu, int64_t wide_tiles) {
+  const int mode = mid_mode(M, W);
+  float c = 0.0f;
+  if (mode < 0 || best_tile(mode, M, W.rows, glu, false, &c) == kNoTile) return false;
+  const int64_t n = cus(), full = wide_tiles / n, rest = wide_tiles % n;
+  return c < kWideStep[mode] * float(full + (rest ? 1 : 0));
+}
+
+bool launch_gemm_mid(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi, float *C,
+                     _Float16 *C16, _Float16 *C16lo, int ldc, const float *bias, hipStream_t st, const _Float16 *ks) {
+  const int mode = mid_mode(M, W);
+  if (mode < 0 || !A || !Alo) return false;
+  const bool glu = epi == Epi::SWIGLU || epi == Epi::GEGLU, f16_only = epi == Epi::GEGLU || epi == Epi::RELU16;
+  if (epi == Epi::F16 || (f16_only && mode != W1)) return false;
+  LG_REQUIRE(mode != WQ4 || ks, "gemm: an exact Q4_K launch needs its activation's chunk sums");
+  float c = 0.0f;
+  const int tile = best_tile(mode, M, W.rows, glu, false, &c);
+  if (tile == kNoTile) return false;
+  const RopeKvOut none;
+  const Launch l{A, Alo, M, W, C, C16, C16lo, ldc, bias, none, st, ks};
+  switch (epi) {
+    case Epi::F32: launch_mode<int(Epi::F32)>(mode, tile, l); break;
+    case Epi::ADD: launch_mode<int(Epi::ADD)>(mode, tile, l); break;
+    case Epi::SWIGLU: launch_mode<int(Epi::SWIGLU)>(mode, tile, l); break;
+    case Epi::GEGLU: launch_mode<int(Epi::GEGLU)>(mode, tile, l); break;
+    case Epi::RELU16: launch_mode<int(Epi::RELU16)>(mode, tile, l); break;
+    default: return false;
+  }
+  return true;
+}
+
+bool gemm_mid_rope_takes(int M, const DevMatrix &W, int hd) {
+  return (hd == 64 || hd == 128) && W.rows % hd == 0 && mid_mode(M, W) >= 0;
+}
+
+void launch_gemm_mid_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, const float *bias,
+                          const RopeKvOut &ro, hipStream_t st, const _Float16 *ks) {
+  LG_REQUIRE(A && Alo && gemm_mid_rope_takes(M, W, ro.hd) && ro.col0 % ro.hd == 0 &&
+                 ro.col0 / ro.hd + W.rows / ro.hd <= ro.hq + 2 * ro.hkv,
+             "gemm rope: %d rows of this projection are not a launch of the 64-column tiles", M);
+  LG_REQUIRE(ro.cosT && ro.sinT && ro.tok_pos && ro.tok_page && ro.q16 && ro.q16lo && ro.kpool && ro.vpool,
+             "gemm rope: missing output");
+  LG_REQUIRE(ro.page_tokens >= 4 && ro.page_tokens % 4 == 0 && ro.page_stride > 0, "gemm rope: bad page geometry");
+  LG_REQUIRE(ro.kv_planes == 1 || ro.kv_planes == 2, "gemm rope: KV pools hold 1 or 2 planes, not %d", ro.kv_planes);
+  const int mode = mid_mode(M, W);
+  LG_REQUIRE(mode != WQ4 || ks, "gemm: an exact Q4_K launch needs its activation's chunk sums");
+  float c = 0.0f;
+  const int tile = best_tile(mode, M, W.rows, false, true, &c);
+  launch_mode<kTileEpiRope>(mode, tile, Launch{A, Alo, M, W, nullptr, nullptr, nullptr, 0, bias, ro, st, ks});
+}
+
+bool gemm_mid_laya_rope_takes(int M, const DevMatrix &W) { return W.rows % 64 == 0 && mid_mode(M, W) == W1; }
+
+void launch_gemm_mid_laya_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, const float *bias,
+                               const float *cosT, const float *sinT, const int32_t *tok_pos, int heads, float *C,
+                               int ldc, hipStream_t st) {
+  LG_REQUIRE(A && Alo && C && cosT && sinT && tok_pos, "gemm laya rope: missing operand");
+  LG_REQUIRE(gemm_mid_laya_rope_takes(M, W) && heads > 0 && W.rows == 3 * heads * 64 && ldc >= W.rows,
+             "gemm laya rope: %d rows are not q|k|v of %d 64-dim heads", W.rows, heads);
+  RopeKvOut ro;
+  ro.cosT = cosT;
+  ro.sinT = sinT;
+  ro.tok_pos = tok_pos;
+  ro.hq = heads;
+  ro.hd = 64;
+  float c = 0.0f;
+  const int tile = best_tile(W1, M, W.rows, false, true, &c);
+  launch_mode<kTileEpiLayaRope>(W1, tile, Launch{A, Alo, M, W, C, nullptr, nullptr, ldc, bias, ro, st, nullptr});
+}
+
+}  // namespace lg

@@ -33,13 +33,6 @@ bool launch_gemm_q8_exact(const _Float16 *A, const _Float16 *Alo, int M, const D
   return launch_cfg<LG_Q8_0, SPLIT, 64, 4, 4, 1>(A, Alo, M, W, epi, C, C16, C16lo, ldc, bias, st);
 }
 
-bool launch_gemm_q8_small_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, const float *bias,
-                               const RopeKvOut &ro, hipStream_t st) {
-  const bool ok = launch_cfg_rope<LG_Q8_0, SPLIT, 128, 1, 2>(A, Alo, M, W, bias, ro, st);
-  if (ok) HIP_CHECK(hipGetLastError());
-  return ok;
-}
-
 bool launch_gemm_q4_exact(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi,
                           float *C, _Float16 *C16, _Float16 *C16lo, int ldc, const float *bias,
                           hipStream_t st, const _Float16 *ks) {
@@ -60,7 +53,6 @@ bool launch_gemm_q4_exact(const _Float16 *A, const _Float16 *Alo, int M, const D
   return launch_cfg<LG_Q4_K, SPLIT, 64, 4, 4, 1>(A, Alo, M, W, epi, C, C16, C16lo, ldc, bias, st, ks);
 }
 
-namespace {
 int device_cus() {
   static thread_local int dev = -1, cus = 0;
   int d = 0;
@@ -71,30 +63,14 @@ int device_cus() {
   }
   return cus;
 }
-}  // namespace
 
 namespace {
 // the wide kernel's mode for W, or -1 when it does not take an M-row launch of W with epilogue
 // EPI (an Epi value or wide::kEpiRopeKv)
 int wide_mode(int M, const DevMatrix &W, int EPI) {
   using namespace wide;
-  if (M <= 0 || !W.pc) return -1;
-  int mode;
-  switch (W.kind) {
-    case LG_Q8_0: mode = WQ8; if (!W.pcs) return -1; break;
-    case LG_F16: mode = W1; break;
-    case LG_Q4_K:  // the two-pass copy (codes, scales, correction planes), or hi/lo planes
-      if (needs_ksum(W)) {
-        mode = WQ4;
-        if (!W.pcs || !W.pcl) return -1;
-      } else {
-        mode = W2;
-        if (!W.pcl) return -1;
-      }
-      break;
-    case LG_Q6_K: mode = W2; if (!W.pcl) return -1; break;
-    default: return -1;
-  }
+  const int mode = prefill_mode(W);
+  if (M <= 0 || mode < 0) return -1;
   if (EPI != int(Epi::F32) && EPI != int(Epi::ADD) && EPI != int(Epi::SWIGLU) && EPI != int(Epi::GEGLU) &&
       EPI != kEpiRopeKv && EPI != kEpiLayaRope)
     return -1;
@@ -103,11 +79,12 @@ int wide_mode(int M, const DevMatrix &W, int EPI) {
   if (K % BK != 0 || N % BN != 0) return -1;  // gated: 128 gate + 128 up rows a tile
   const int NT = glu ? (N / 2) / (BN / 2) : N / BN;
   if (int64_t(N) * K * 2 >= (int64_t(1) << 32)) return -1;  // 32-bit buffer offsets of the weights
-  // fewer 256 x 256 tiles than 5/8 of the CUs leaves too many idle: the 128 x 128 tiles fill the device
-  // better.  Between that and one tile per CU the 256 x 256 tiles still win (F16 at 1437 rows x 7168 gated,
-  // 168 tiles: 50.3 against 60.0 us; 2048 x 6144, 192 tiles: 91.7 against 120.4; 3000 x 5120, 240 tiles:
-  // 57.1 against 77.2), and below it they lose (1437 x 5120, 120 tiles: 48.1 against 41.8)
-  if (int64_t((M + BM - 1) / BM) * NT * 8 < int64_t(device_cus()) * 5) return -1;
+  // fewer 256 x 256 tiles than 5/8 of the CUs leaves too many idle: the smaller tiles fill the device better.  Between
+  // that and one tile per CU the 256 x 256 tiles still win (F16 at 1437 rows x 7168 gated, 168 tiles: 47.8 us against
+  // 53.4 of gemm_mid.h's best), and below it they lose.  A last round that is nearly empty loses too (301 rows x 37888
+  // gated F16, 296 tiles, against 170 us): gemm_mid_ahead compares the rounds.
+  const int64_t tiles = int64_t((M + BM - 1) / BM) * NT;
+  if (tiles * 8 < int64_t(device_cus()) * 5 || gemm_mid_ahead(M, W, glu, tiles)) return -1;
   return mode;
 }
 

@@ -187,13 +187,20 @@ bool gemm_wide_takes(int M, const DevMatrix &W, Epi epi);
 void launch_gemm_wide_laya_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, const float *bias,
                                 const float *cosT, const float *sinT, const int32_t *tok_pos, int heads, float *C,
                                 int ldc, hipStream_t st, const _Float16 *ks = nullptr);
-// Short launches (fewer than 128 tiles of 64 x 64) of an F16 or Q8_0 q|k|v projection in the exact
-// split mode: the 32-row tile GEMM with the same rotating epilogue as launch_gemm_wide_rope (head_dim
-// 64 or 128, ro.col0 a multiple of it), the same bits as the F32 GEMM followed by the RoPE kernel.
-// gemm_small_rope_takes tells whether launch_gemm_small_rope launches (it returns false otherwise).
-bool gemm_small_rope_takes(int M, const DevMatrix &W, int hd);
-bool launch_gemm_small_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, const float *bias,
-                            const RopeKvOut &ro, hipStream_t st);
+// Compute units of the current device.
+int device_cus();
+// Whether the smaller tiles of gemm_mid.h are ahead of `wide_tiles` 256 x 256 tiles for M rows of W.
+bool gemm_mid_ahead(int M, const DevMatrix &W, bool glu, int64_t wide_tiles);
+// The two rotating q|k|v launches above on the tiles of gemm_mid.h, for any M the 256 x 256 GEMM does not take, in the
+// exact split mode: the same bits as the F32 GEMM followed by the RoPE kernel.  head_dim 64 or 128, ro.col0 a
+// multiple of it; anything the takes function refuses fails.  The encoder's needs F16 weights.
+bool gemm_mid_rope_takes(int M, const DevMatrix &W, int hd);
+void launch_gemm_mid_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, const float *bias,
+                          const RopeKvOut &ro, hipStream_t st, const _Float16 *ks = nullptr);
+bool gemm_mid_laya_rope_takes(int M, const DevMatrix &W);
+void launch_gemm_mid_laya_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, const float *bias,
+                               const float *cosT, const float *sinT, const int32_t *tok_pos, int heads, float *C,
+                               int ldc, hipStream_t st);
 
 // RoPE on q and k of q|k|v rows ((hq+2hkv)*hd f32) with tables cos/sin[ctx][hd], q written
 // out, k and v written into the K page rows [hkv][page_tokens][hd] and V page columns
