@@ -772,8 +772,12 @@ BatchPlan *Engine::batch_create(const lg_request *reqs, int nreq) {
       if (!fresh) max_pages = std::max(max_pages, (s.len + q.n + 63) / 64);
       max_len = std::max(max_len, s.len + q.n);
     }
-    const int gtiles = arch == Arch::Decoder ? attn_prefill_group_tiles(hq, hkv, max_len) : 4;
-    b->gtiles = gtiles;
+    if (arch == Arch::Decoder) {
+      std::vector<int32_t> fresh_n;
+      for (int r = 0; r < nreq; ++r) fresh_n.push_back(reqs[r].n);
+      b->tiling = attn_prefill_tiling(hq, hkv, max_len, fresh_n.data(), nreq);
+    }
+    const int gtiles = b->tiling.group_tiles, trows = b->tiling.tile_rows;
     const int64_t T = std::accumulate(reqs, reqs + nreq, int64_t(0), [](int64_t a, const lg_request &q) { return a + q.n; });
     if (T > max_batch_tokens_) fail(LG_ERR_INVALID, "batch of %lld tokens exceeds max_batch_tokens %lld", (long long)T, (long long)max_batch_tokens_);
     // reserve pages (all or nothing)
@@ -803,17 +807,17 @@ BatchPlan *Engine::batch_create(const lg_request *reqs, int nreq) {
       // attention groups of <= gtiles consecutive tiles, cut from the request's end and listed last
       // first: the leftover short group is the one nearest the start (the fewest pages), not a
       // group of one or two tiles that reads every page with most of its waves idle
-      const int t_first = int(tiles_s.size()), ntl = (q.n + 31) / 32;
+      const int t_first = int(tiles_s.size()), ntl = (q.n + trows - 1) / trows;
       for (int e = ntl; e > 0; e -= gtiles) {
         const int b = std::max(0, e - gtiles);
         grp_f.push_back(t_first + b);
         grp_c.push_back(e - b);
       }
-      for (int i = 0; i < q.n; i += 32) {
+      for (int i = 0; i < q.n; i += trows) {
         tiles_s.push_back(r);
         tiles_r.push_back(row + i);
         tiles_p.push_back(s.len + i);
-        tiles_n.push_back(std::min(32, q.n - i));
+        tiles_n.push_back(std::min(trows, q.n - i));
       }
       if (ot)  // attention work of a fresh sequence: 16 query rows x key ranges of <= 256
         for (int i = 0; i < q.n; i += 16) {
@@ -974,7 +978,7 @@ void Engine::run_layers_prefill(BatchPlan &b, lg_cancel_fn cancel, void *arg) {
     prof.begin("attn_prefill", stream);
     launch_attn_prefill(q16, q16lo, T, hq, g, kpool(l), vpool(l), b.pages, b.max_pages, b.tile_seq,
                         b.tile_row0, b.tile_pos0, b.tile_n, b.ntiles, b.grp_first, b.grp_count,
-                        b.ngroups, b.gtiles, att, attlo, stream);
+                        b.ngroups, b.tiling, att, attlo, stream);
     prof.end(0, 0, stream);
     gemm(att, attlo, T, ly.wo, Epi::ADD, x, nullptr, nullptr, d, nullptr);
     prof.begin("rmsnorm", stream);

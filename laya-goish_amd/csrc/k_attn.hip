@@ -86,7 +86,10 @@ __device__ __forceinline__ half8 lds_half8(const unsigned char *base, int slot) 
 // up to 8 waves per CU: 128 KiB of LDS at head_dim 128).  1: each page is loaded, then consumed, and
 // two workgroups of 4 waves share a CU, one computing while the other waits for its page (the short
 // sequences, where a workgroup's start and its few pages' waits dominate).
-template <int HD, int NQ, int NKV, int W, int GB, int STG>
+// QB: 16-query blocks of a wave's tile (tiles of 16 QB rows).  2: each operand read from LDS feeds two blocks.  1: when
+// tiles of 32 rows make too few workgroups to fill the device (single requests), twice the waves with half the
+// work per page each; a query's arithmetic is the same.
+template <int HD, int NQ, int NKV, int W, int GB, int STG, int QB>
 __global__ __launch_bounds__(64 * W, STG == 1 ? 2 : 1) void attn_prefill_kernel(
     const _Float16 *__restrict__ q16, const _Float16 *__restrict__ q16lo, int hq, KvGeom g,
     const _Float16 *__restrict__ kpool, const _Float16 *__restrict__ vpool, const int32_t *__restrict__ pages,
@@ -164,9 +167,9 @@ __global__ __launch_bounds__(64 * W, STG == 1 ? 2 : 1) void attn_prefill_kernel(
 
   // queries qb * 16 + lr of the tile (rows past n repeat row n - 1 and are never stored), the eight
   // dims 32 c + 8 g .. + 8 of each 32-deep chunk c
-  half8 qr[2][NC], ql[2][NQ == 2 ? NC : 1];
+  half8 qr[QB][NC], ql[QB][NQ == 2 ? NC : 1];
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
+  for (int qb = 0; qb < QB; ++qb) {
     const int64_t qo = int64_t(row0 + min(qb * 16 + lr, n - 1)) * qw + h * HD + qg * 8;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -174,14 +177,19 @@ __global__ __launch_bounds__(64 * W, STG == 1 ? 2 : 1) void attn_prefill_kernel(
       if constexpr (NQ == 2) ql[qb][c] = *reinterpret_cast<const half8 *>(q16lo + qo + 32 * c);
     }
   }
-  f32x4 acc[2][DB];
+  f32x4 acc[QB][DB];
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
+  for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
     for (int b = 0; b < DB; ++b)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[qb][b][r] = 0.0f;
-  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.0f, 0.0f};
+  float m[QB], l[QB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    m[qb] = -INFINITY;
+    l[qb] = 0.0f;
+  }
   const int npages = glast / P + 1;
   const int mypages = active ? (pos0 + n - 1) / P + 1 : 0;
   // this lane's K operand rows: key ck * 32 + 8 (lr / 4) + 4 h + lr % 4 of block (ck, h); their
@@ -205,9 +213,9 @@ __global__ __launch_bounds__(64 * W, STG == 1 ? 2 : 1) void attn_prefill_kernel(
       const unsigned char *stage = lds + st * S::BYTES;
       const unsigned char *kl_ = stage + S::KPL * 16 * (NKV - 1);  // K lo plane (= hi when NKV 1)
       const unsigned char *vh_ = stage + S::KSLOTS * 16, *vl_ = vh_ + S::VPL * 16 * (NKV - 1);
-      f32x4 s[2][2][2];  // [qb][ck][h]
+      f32x4 s[QB][2][2];  // [qb][ck][h]
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb)
+      for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
         for (int ck = 0; ck < 2; ++ck)
 #pragma unroll
@@ -225,20 +233,20 @@ __global__ __launch_bounds__(64 * W, STG == 1 ? 2 : 1) void attn_prefill_kernel(
             if constexpr (NQ == 2 && NKV == 2) {
               const half8 kl8 = lds_half8(kl_, slot);
 #pragma unroll
-              for (int qb = 0; qb < 2; ++qb) {
+              for (int qb = 0; qb < QB; ++qb) {
                 s[qb][ck][hh] = MFMA(kh8, qr[qb][c], s[qb][ck][hh]);
                 s[qb][ck][hh] = MFMA(kl8, qr[qb][c], s[qb][ck][hh]);
                 s[qb][ck][hh] = MFMA(kh8, ql[qb][c], s[qb][ck][hh]);
               }
             } else if constexpr (NQ == 2) {
 #pragma unroll
-              for (int qb = 0; qb < 2; ++qb) {
+              for (int qb = 0; qb < QB; ++qb) {
                 s[qb][ck][hh] = MFMA(kh8, qr[qb][c], s[qb][ck][hh]);
                 s[qb][ck][hh] = MFMA(kh8, ql[qb][c], s[qb][ck][hh]);
               }
             } else {
 #pragma unroll
-              for (int qb = 0; qb < 2; ++qb) s[qb][ck][hh] = MFMA(kh8, qr[qb][c], s[qb][ck][hh]);
+              for (int qb = 0; qb < QB; ++qb) s[qb][ck][hh] = MFMA(kh8, qr[qb][c], s[qb][ck][hh]);
             }
           }
       // s[qb][ck][h][e] <-> key kt * P + ck * 32 + 8 qg + 4 h + e, query qb * 16 + lr.  The queries
@@ -246,7 +254,7 @@ __global__ __launch_bounds__(64 * W, STG == 1 ? 2 : 1) void attn_prefill_kernel(
       // reaches past the tile's first query needs the causal mask.
       if (kt * P + P - 1 > pos0) {
 #pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
+        for (int qb = 0; qb < QB; ++qb) {
           const int lim = pos0 + qb * 16 + lr - kt * P - 8 * qg;  // mask offsets ck * 32 + 4 h + e above
 #pragma unroll
           for (int ck = 0; ck < 2; ++ck)
@@ -258,7 +266,7 @@ __global__ __launch_bounds__(64 * W, STG == 1 ? 2 : 1) void attn_prefill_kernel(
         }
       }
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) {
+      for (int qb = 0; qb < QB; ++qb) {
         float mt = -INFINITY;
 #pragma unroll
         for (int ck = 0; ck < 2; ++ck)
@@ -304,9 +312,9 @@ __global__ __launch_bounds__(64 * W, STG == 1 ? 2 : 1) void attn_prefill_kernel(
       // of its query, against dims 16 b + lr of V at the same keys
 #pragma unroll
       for (int ck = 0; ck < 2; ++ck) {
-        half8 ph[2], pl[2];
+        half8 ph[QB], pl[QB];
 #pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
+        for (int qb = 0; qb < QB; ++qb) {
           float pv[8];
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
@@ -325,20 +333,20 @@ __global__ __launch_bounds__(64 * W, STG == 1 ? 2 : 1) void attn_prefill_kernel(
           if constexpr (NQ == 2 && NKV == 2) {
             const half8 vl = lds_half8(vl_, vo);
 #pragma unroll
-            for (int qb = 0; qb < 2; ++qb) {
+            for (int qb = 0; qb < QB; ++qb) {
               acc[qb][b] = MFMA(vh, ph[qb], acc[qb][b]);
               acc[qb][b] = MFMA(vl, ph[qb], acc[qb][b]);
               acc[qb][b] = MFMA(vh, pl[qb], acc[qb][b]);
             }
           } else if constexpr (NQ == 2) {
 #pragma unroll
-            for (int qb = 0; qb < 2; ++qb) {
+            for (int qb = 0; qb < QB; ++qb) {
               acc[qb][b] = MFMA(vh, ph[qb], acc[qb][b]);
               acc[qb][b] = MFMA(vh, pl[qb], acc[qb][b]);
             }
           } else {
 #pragma unroll
-            for (int qb = 0; qb < 2; ++qb) acc[qb][b] = MFMA(vh, ph[qb], acc[qb][b]);
+            for (int qb = 0; qb < QB; ++qb) acc[qb][b] = MFMA(vh, ph[qb], acc[qb][b]);
           }
         }
       }
@@ -355,7 +363,7 @@ __global__ __launch_bounds__(64 * W, STG == 1 ? 2 : 1) void attn_prefill_kernel(
   if (!active) return;
   // acc[qb][b][r] <-> dim 16 b + 4 qg + r of query qb * 16 + lr
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
+  for (int qb = 0; qb < QB; ++qb) {
     if (qb * 16 + lr >= n) continue;
     const float inv = 1.0f / l[qb];
     const int64_t obase = int64_t(row0 + qb * 16 + lr) * qw + h * HD + 4 * qg;
@@ -749,8 +757,16 @@ PrefillShape prefill_shape(int G) {
 constexpr int kShortSeq = 1024;
 }  // namespace
 
-int attn_prefill_group_tiles(int hq, int hkv, int max_len) {
-  return hq == hkv && max_len <= kShortSeq ? 4 : prefill_shape(hq / hkv).t;
+AttnTiling attn_prefill_tiling(int hq, int hkv, int max_len, const int32_t *new_tokens, int nseq) {
+  const PrefillShape sh = prefill_shape(hq / hkv);
+  const AttnTiling big{32, hq == hkv && max_len <= kShortSeq ? 4 : sh.t};
+  int64_t groups = 0;
+  for (int i = 0; i < nseq; ++i) groups += (new_tokens[i] + 32 * big.group_tiles - 1) / (32 * big.group_tiles);
+  // fewer workgroups of 32-row tiles than CUs: 16-row tiles, one head block of at most eight waves a workgroup (one
+  // request of 144 tokens, 8 heads of 64: 13.0 -> 9.6 us; 301 tokens, 16 heads of 128: 26.0 -> 17.8; 700 tokens, 28
+  // heads over 4: 48.1 -> 31.3)
+  if (groups * hkv * (hq / hkv / sh.gb) < device_cus()) return {16, sh.gb == 1 ? 4 : sh.t};
+  return big;
 }
 
 void launch_attn_prefill(const _Float16 *q16, const _Float16 *q16_lo, int T, int hq,
@@ -758,7 +774,7 @@ void launch_attn_prefill(const _Float16 *q16, const _Float16 *q16_lo, int T, int
                          const int32_t *pages, int max_pages, const int32_t *tile_seq,
                          const int32_t *tile_row0, const int32_t *tile_pos0,
                          const int32_t *tile_n, int ntiles, const int32_t *grp_first,
-                         const int32_t *grp_count, int ngroups, int group_tiles, _Float16 *out16,
+                         const int32_t *grp_count, int ngroups, AttnTiling tiling, _Float16 *out16,
                          _Float16 *out16_lo, hipStream_t st) {
   LG_REQUIRE(g.page_tokens == P, "attention: page size must be %d", P);
   LG_REQUIRE(g.hkv > 0 && hq % g.hkv == 0, "attention: hq %% hkv != 0");
@@ -768,28 +784,35 @@ void launch_attn_prefill(const _Float16 *q16, const _Float16 *q16_lo, int T, int
   LG_REQUIRE(!split || out16_lo, "attention: split path needs the lo output plane");
   LG_REQUIRE(grp_first && grp_count && ngroups > 0 && ngroups <= ntiles, "attention: bad tile groups");
   const int G = hq / g.hkv;
-  const bool single = G == 1 && group_tiles == 4;  // attn_prefill_group_tiles' short-sequence form
-  const PrefillShape sh = single ? PrefillShape{1, 4} : prefill_shape(G);
-  LG_REQUIRE(group_tiles == sh.t, "attention: groups of %d tiles, kernel shape of %d", group_tiles, sh.t);
+  const bool small = tiling.tile_rows == 16;
+  const bool single = !small && G == 1 && tiling.group_tiles == 4;  // attn_prefill_tiling's short-sequence form
+  PrefillShape sh = prefill_shape(G);
+  if (single || (small && sh.gb == 1)) sh = {1, 4};
+  LG_REQUIRE((small || tiling.tile_rows == 32) && tiling.group_tiles == sh.t,
+             "attention: groups of %d tiles of %d rows, kernel shape of %d", tiling.group_tiles, tiling.tile_rows, sh.t);
   const int64_t nwg = int64_t(ngroups) * g.hkv * (G / sh.gb);
   LG_REQUIRE(nwg < (1ll << 31), "attention: too many tiles");
   const dim3 grid{static_cast<uint32_t>(nwg)}, block{static_cast<uint32_t>(64 * sh.gb * sh.t)};
   const _Float16 *kp = static_cast<const _Float16 *>(kpool), *vp = static_cast<const _Float16 *>(vpool);
-#define LAUNCH(HDV, NQV, NKVV, WV, GBV, STGV)                                                             \
-  hipLaunchKernelGGL((attn_prefill_kernel<HDV, NQV, NKVV, WV, GBV, STGV>), grid, block, 0, st, q16, q16_lo, hq, g, kp, vp, \
-                     pages, max_pages, grp_first, grp_count, tile_seq, tile_row0, tile_pos0, tile_n, out16,    \
-                     out16_lo)
+#define LAUNCH(HDV, NQV, NKVV, WV, GBV, STGV, QBV)                                                             \
+  hipLaunchKernelGGL((attn_prefill_kernel<HDV, NQV, NKVV, WV, GBV, STGV, QBV>), grid, block, 0, st, q16, q16_lo, hq, g, \
+                     kp, vp, pages, max_pages, grp_first, grp_count, tile_seq, tile_row0, tile_pos0, tile_n,    \
+                     out16, out16_lo)
+#define GROUPED(HDV, NQV, NKVV, QBV)                                           \
+  switch (sh.gb) {                                                             \
+    case 2: LAUNCH(HDV, NQV, NKVV, 8, 2, 2, QBV); break;                       \
+    case 4: LAUNCH(HDV, NQV, NKVV, 8, 4, 2, QBV); break;                       \
+    case 7: LAUNCH(HDV, NQV, NKVV, 7, 7, 2, QBV); break;                       \
+    case 8: LAUNCH(HDV, NQV, NKVV, 8, 8, 2, QBV); break;                       \
+    default: LAUNCH(HDV, NQV, NKVV, QBV == 1 ? 4 : 8, 1, 2, QBV); break;       \
+  }
 #define SHAPES(HDV, NQV, NKVV)                                                 \
-  if (single) {                                                                \
-    LAUNCH(HDV, NQV, NKVV, 4, 1, 1);                                           \
+  if (small) {                                                                 \
+    GROUPED(HDV, NQV, NKVV, 1)                                                 \
+  } else if (single) {                                                         \
+    LAUNCH(HDV, NQV, NKVV, 4, 1, 1, 2);                                        \
   } else {                                                                     \
-    switch (sh.gb) {                                                           \
-      case 2: LAUNCH(HDV, NQV, NKVV, 8, 2, 2); break;                          \
-      case 4: LAUNCH(HDV, NQV, NKVV, 8, 4, 2); break;                          \
-      case 7: LAUNCH(HDV, NQV, NKVV, 7, 7, 2); break;                          \
-      case 8: LAUNCH(HDV, NQV, NKVV, 8, 8, 2); break;                          \
-      default: LAUNCH(HDV, NQV, NKVV, 8, 1, 2); break;                         \
-    }                                                                          \
+    GROUPED(HDV, NQV, NKVV, 2)                                                 \
   }
   if (g.hd == 128) {
     if (g.split) { SHAPES(128, 2, 2) } else if (split) { SHAPES(128, 2, 1) } else { SHAPES(128, 1, 1) }
@@ -799,6 +822,7 @@ void launch_attn_prefill(const _Float16 *q16, const _Float16 *q16_lo, int T, int
     fail(LG_ERR_UNSUPPORTED, "attention: head_dim %d not supported (64, 128)", g.hd);
   }
 #undef SHAPES
+#undef GROUPED
 #undef LAUNCH
   HIP_CHECK(hipGetLastError());
 }

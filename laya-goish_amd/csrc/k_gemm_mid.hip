@@ -23,30 +23,32 @@ struct StepCost {
 };
 constexpr StepCost kCost[4][kTiles] = {
     /* WQ8 */ {{0.24f, 0.40f}, {0.31f, 0.54f}, {0.46f, 0.78f}, {0.84f, 1.03f}, {0.70f, 1.40f}, {1.11f, 2.25f}},
-    /* W1  */ {{0.20f, 0.36f}, {0.24f, 0.47f}, {0.36f, 0.70f}, {0.80f, 0.92f}, {0.57f, 1.14f}, {0.95f, 1.90f}},
+    /* W1  */ {{0.20f, 0.36f}, {0.24f, 0.47f}, {0.36f, 0.70f}, {0.80f, 0.95f}, {0.57f, 1.14f}, {0.95f, 1.90f}},
     /* W2  */ {{0.27f, 0.50f}, {0.43f, 0.86f}, {0.49f, 0.98f}, {0, 0}, {0.85f, 1.70f}, {1.50f, 3.00f}},
     /* WQ4 */ {{0.24f, 0.40f}, {0.31f, 0.54f}, {0.46f, 0.78f}, {0, 0}, {0.70f, 1.40f}, {1.11f, 2.25f}},
 };
 constexpr int kHM[kTiles] = {1, 1, 2, 2, 2, 4}, kHN[kTiles] = {1, 2, 2, 4, 4, 4};
-// a 256 x 256 tile's microseconds per 64-deep step, one workgroup per CU (mode order as above)
-constexpr float kWideStep[4] = {3.6f, 3.0f, 4.9f, 3.6f};
+// a 256 x 256 tile's microseconds per 64-deep step, one workgroup per CU (mode order as above; F16 at 168 and 198 tiles
+// of K 1024, the others from full rounds)
+constexpr float kWideStep[4] = {3.5f, 2.75f, 4.7f, 3.5f};
 
-int cus() { return device_cus(); }
-
-// Rounds of two workgroups per CU, the last one alone when half a round or less is left.
-float cost(const StepCost &c, int64_t tiles) {
-  const int64_t n = cus(), rounds = tiles / (2 * n), rest = tiles - rounds * 2 * n;
-  return float(rounds) * c.two + (rest == 0 ? 0.0f : rest <= n ? c.one : c.two);
+// Microseconds of `nk` steps: rounds of two workgroups per CU, the last one alone when half a round or less is left, each
+// with the fill and drain of its pipeline.
+constexpr float kRound = 2.0f;
+float cost(const StepCost &c, int64_t tiles, int nk) {
+  const int64_t n = device_cus(), rounds = tiles / (2 * n), rest = tiles - rounds * 2 * n;
+  return float(rounds) * (c.two * nk + kRound) + (rest == 0 ? 0.0f : (rest <= n ? c.one : c.two) * nk + kRound);
 }
 
 // The cheapest configuration for M rows of a matrix of `rows` weight rows (only those of 64 columns when rope), and
 // its cost; kNoTile when none divides the output.
-int best_tile(int mode, int M, int rows, bool glu, bool rope, float *best) {
+int best_tile(int mode, int M, const DevMatrix &W, bool glu, bool rope, float *best) {
+  const int rows = W.rows;
   int t = kNoTile;
   for (int i = 0; i < kTiles; ++i) {
     const int bm = 32 * kHM[i], bn = 32 * kHN[i];
     if (kCost[mode][i].one == 0 || rows % bn || (glu && kHN[i] % 2) || (rope && kHN[i] != 2)) continue;
-    const float c = cost(kCost[mode][i], int64_t((M + bm - 1) / bm) * (rows / bn));
+    const float c = cost(kCost[mode][i], int64_t((M + bm - 1) / bm) * (rows / bn), W.cols / mid::BK);
     if (t == kNoTile || c < *best) {
       t = i;
       *best = c;
@@ -158,9 +160,9 @@ void launch_mode(int mode, int tile, const Launch &l) {
 bool gemm_mid_ahead(int M, const DevMatrix &W, bool glu, int64_t wide_tiles) {
   const int mode = mid_mode(M, W);
   float c = 0.0f;
-  if (mode < 0 || best_tile(mode, M, W.rows, glu, false, &c) == kNoTile) return false;
-  const int64_t n = cus(), full = wide_tiles / n, rest = wide_tiles % n;
-  return c < kWideStep[mode] * float(full + (rest ? 1 : 0));
+  if (mode < 0 || best_tile(mode, M, W, glu, false, &c) == kNoTile) return false;
+  const int64_t rounds = (wide_tiles + device_cus() - 1) / device_cus();
+  return c < float(rounds) * (kWideStep[mode] * (W.cols / mid::BK) + kRound);
 }
 
 bool launch_gemm_mid(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi, float *C,
@@ -171,7 +173,7 @@ bool launch_gemm_mid(const _Float16 *A, const _Float16 *Alo, int M, const DevMat
   if (epi == Epi::F16 || (f16_only && mode != W1)) return false;
   LG_REQUIRE(mode != WQ4 || ks, "gemm: an exact Q4_K launch needs its activation's chunk sums");
   float c = 0.0f;
-  const int tile = best_tile(mode, M, W.rows, glu, false, &c);
+  const int tile = best_tile(mode, M, W, glu, false, &c);
   if (tile == kNoTile) return false;
   const RopeKvOut none;
   const Launch l{A, Alo, M, W, C, C16, C16lo, ldc, bias, none, st, ks};
@@ -202,7 +204,7 @@ void launch_gemm_mid_rope(const _Float16 *A, const _Float16 *Alo, int M, const D
   const int mode = mid_mode(M, W);
   LG_REQUIRE(mode != WQ4 || ks, "gemm: an exact Q4_K launch needs its activation's chunk sums");
   float c = 0.0f;
-  const int tile = best_tile(mode, M, W.rows, false, true, &c);
+  const int tile = best_tile(mode, M, W, false, true, &c);
   launch_mode<kTileEpiRope>(mode, tile, Launch{A, Alo, M, W, nullptr, nullptr, nullptr, 0, bias, ro, st, ks});
 }
 
@@ -221,7 +223,7 @@ void launch_gemm_mid_laya_rope(const _Float16 *A, const _Float16 *Alo, int M, co
   ro.hq = heads;
   ro.hd = 64;
   float c = 0.0f;
-  const int tile = best_tile(W1, M, W.rows, false, true, &c);
+  const int tile = best_tile(W1, M, W, false, true, &c);
   launch_mode<kTileEpiLayaRope>(W1, tile, Launch{A, Alo, M, W, C, nullptr, nullptr, ldc, bias, ro, st, nullptr});
 }
 

@@ -215,22 +215,25 @@ void launch_rope_kv_tiles(const float *qkv, int hq, const KvGeom &g, const float
                           void *kpool, void *vpool, hipStream_t st);
 
 // Causal prefill attention over the paged cache, queries as launch_rope_kv_tiles leaves them
-// (pre-scaled by log2(e) / sqrt(hd)).  Work items: tiles of 32 query rows of one
+// (pre-scaled by log2(e) / sqrt(hd)).  Work items: tiles of at most tiling.tile_rows query rows of one
 // sequence (tile_seq, tile_row0 = first batch row, tile_pos0 = its position, tile_n rows).
 // q16_lo != nullptr selects the split-precision path, over the split cache (g.split) or an f16
 // one; the output is then written as hi/lo planes (out16, out16_lo).  f16 queries need the f16
-// cache.  Tiles go in groups (grp_first[i],
-// grp_count[i] for i < ngroups) of at most group_tiles = attn_prefill_group_tiles(hq, hkv, max_len)
-// consecutive tiles of one sequence (max_len: the longest sequence of the batch, its own tokens
-// included); each group's workgroups share every K/V page through LDS.  head_dim 64 or 128.
-// A query's output does not depend on which group or batch its tile is in.
-int attn_prefill_group_tiles(int hq, int hkv, int max_len);
+// cache.  Tiles go in groups (grp_first[i], grp_count[i] for i < ngroups) of at most tiling.group_tiles
+// consecutive tiles of one sequence; each group's workgroups share every K/V page through LDS.  head_dim 64 or 128.
+// A query's output does not depend on which tiling, group or batch it is in.
+struct AttnTiling {
+  int tile_rows = 32, group_tiles = 4;
+};
+// The tiling of a batch whose sequences get new_tokens[i] tokens each (max_len: the longest sequence of the batch, its
+// own tokens included).
+AttnTiling attn_prefill_tiling(int hq, int hkv, int max_len, const int32_t *new_tokens, int nseq);
 void launch_attn_prefill(const _Float16 *q16, const _Float16 *q16_lo, int T, int hq,
                          const KvGeom &g, const void *kpool, const void *vpool,
                          const int32_t *pages, int max_pages, const int32_t *tile_seq,
                          const int32_t *tile_row0, const int32_t *tile_pos0,
                          const int32_t *tile_n, int ntiles, const int32_t *grp_first,
-                         const int32_t *grp_count, int ngroups, int group_tiles, _Float16 *out16,
+                         const int32_t *grp_count, int ngroups, AttnTiling tiling, _Float16 *out16,
                          _Float16 *out16_lo, hipStream_t st);
 
 // Decode attention for one new token at position pos of one sequence: q|k|v row `qkv` (before
