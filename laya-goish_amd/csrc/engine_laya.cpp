@@ -253,8 +253,8 @@ void Engine::run_laya(BatchPlan &b, const int32_t *qtype_dev, lg_cancel_fn cance
     }
     prof.begin("laya_attn", stream);
     if (rope && !fused) launch_laya_rope(qkv, T, d, hd, cosT, sinT, b.tok_pos, stream);
-    launch_laya_attn(qkv, d, hd, y.full ? -1 : 64, b.tile_row0, b.tile_pos0, b.tile_n, b.tile_seq, b.seq_n, b.ntiles,
-                     att, attlo, stream);
+    launch_laya_attn(qkv, d, hd, y.full ? -1 : 64, b.tile_row0, b.tile_pos0, b.tile_n, b.tile_seq, b.seq_n, b.grp_first,
+                     b.grp_count, b.ngroups, att, attlo, stream);
     prof.end(0, 0, stream);
     gemm(att, attlo, T, y.wo.w, Epi::ADD, h, nullptr, nullptr, d, y.wo.b);
   };

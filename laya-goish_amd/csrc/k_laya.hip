@@ -118,191 +118,245 @@ __global__ __launch_bounds__(kT) void laya_rope_kernel(float *__restrict__ qkv, 
   }
 }
 
-// Bidirectional attention over q|k|v rows [T][3d] (f32, q and k already rotated), head dim 64,
-// on v_mfma_f32_16x16x16_f16 with every f32 operand split into f16 hi + lo parts and three
-// products per pair (lo*hi, hi*lo, hi*hi; the lo*lo term is below f32 rounding), f32
-// accumulation.  One workgroup per (16 query rows of
-// one sequence, head); its four waves split the visible keys into four ranges of 16-key blocks
-// and merge their (m, l, O) in LDS at the end.  Keys j with |i - j| <= window (window < 0: the
-// whole sequence); scores q.k * (1/sqrt(64)); online softmax in f32 (base 2).  Output f16
-// planes [T][d].
-//   S = Q K^T per block: lane (li = l%16, kg = l/16) supplies Q[li][16g + 4kg + c], c < 4, as the
-//   A operand of k-step g (a permutation of the 64-dim contraction, applied to K alike); operands
-//   come straight from the q|k|v rows as float4 loads, the next block's K and V prefetched in
-//   registers.
-//   D layout: lane l holds S[4kg + r][li], r < 4.  P goes through LDS into the A layout
-//   (P[li][4kg + c]); O += P V with V[4kg + c][16b + li], c < 4, as the B operand.
-constexpr int kPp = 20;  // padded row of a wave's P block [16 rows][16 keys]
-// scores are kept as log2(e) q.k / 8 and exponentiated with the hardware exp2 (v_exp_f32,
-// ~1 ulp): softmax is invariant to the base, and exp2 of a difference costs one instruction
+// Bidirectional attention over q|k|v rows [T][3d] (f32, q and k already rotated), head dim 64, on
+// v_mfma_f32_16x16x32_f16 with every f32 operand split into f16 hi + lo parts and three products per pair (hi.hi,
+// lo.hi, hi.lo; lo.lo is below f32 rounding), f32 accumulation.  Keys j with |i - j| <= window (window < 0: the whole
+// sequence); scores q.k / sqrt(64) in base 2; online softmax in f32.  Output f16 planes [T][d].
+//
+// One workgroup per (group of at most four consecutive 32-row tiles of one sequence, head): its four waves walk the same
+// 64-key blocks (aligned to the sequence's start, so a query's arithmetic depends on its position only), and each
+// block's K and V rows are read, split and staged in LDS once for up to 128 queries, V transposed, the next block's rows
+// on their way in registers.  (The former form gave every 16 queries a workgroup that read and split all keys
+// again, on the 16x16x16 instruction: 699 us a full and ~380 a windowed layer of 64 inputs of 473-512 tokens, against 210
+// and ~165.)  QB 16-query blocks a wave: 2, a wave takes a tile; 1, half a tile, two workgroups (z) a group, when whole
+// groups would leave CUs idle.
+// S^T = K Q^T in 16 x 16 blocks: lane l feeds row lr = l % 16 of key block (ck, hh), which is key ck * 32 + 8 (lr / 4) + 4 hh +
+// lr % 4, so that it receives, for query lr, keys ck * 32 + 8 qg + 4 hh + 0..3, qg = l / 16: blocks (ck, 0) and (ck, 1)
+// together are the eight keys its P^T operand of O^T = V^T P^T takes (the decoder's prefill attention has the same form).
+// LDS: 16-byte chunk x of a K row at slot x ^ kswz(row); V rows (one dim, 64 keys) with one pad slot: operand reads
+// without bank conflicts.
+// scores in base-2 units; applied to them and not to q, whose f16 range stays the operand's own
 constexpr float kScoreLog2 = 0.125f * 1.44269504088896341f;
-constexpr int kOp = 68;  // padded row of a wave's partial O [16 rows][64]
+constexpr int kKB = 64;                     // keys per block
+constexpr int kKSlots = kKB * 8, kVSlots = kHD * 9;  // 16-byte slots of a plane
 
-typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ int laya_kswz(int row) { return (row & 3) | (((row >> 3) & 1) << 2); }
 
-// x = hi + lo with hi = f16(x), lo = f16(x - hi): ~22 significant bits
-__device__ __forceinline__ void split_hl(float4v x, half4v &hi, half4v &lo) {
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    _Float16 h, l;
-    split_f16(x[c], h, l);
-    hi[c] = h;
-    lo[c] = l;
-  }
-}
-
-__device__ __forceinline__ float4v mfma3(half4v ah, half4v al, half4v bh, half4v bl, float4v acc) {
-  acc = __builtin_amdgcn_mfma_f32_16x16x16f16(al, bh, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_16x16x16f16(ah, bl, acc, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x16f16(ah, bh, acc, 0, 0, 0);
-}
-
-struct KVBlock {
-  float4v k[4];
-  float v[16];
-};
-
-__device__ __forceinline__ void laya_load_kv(KVBlock &blk, const float *__restrict__ kbase, int ld, int d, int k0,
-                                             int n, int li, int kg) {
-  const float *kr = kbase + int64_t(min(k0 + li, n - 1)) * ld;
-#pragma unroll
-  for (int g = 0; g < 4; ++g) blk.k[g] = *reinterpret_cast<const float4v *>(kr + 16 * g + 4 * kg);
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const float *vr = kbase + int64_t(min(k0 + 4 * kg + c, n - 1)) * ld + d;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) blk.v[4 * b + c] = vr[16 * b + li];
-  }
-}
-
-__global__ __launch_bounds__(256) void laya_attn_kernel(const float *__restrict__ qkv, int d, int window,
-                                                        const int32_t *__restrict__ tile_row0,
-                                                        const int32_t *__restrict__ tile_pos0,
-                                                        const int32_t *__restrict__ tile_n,
-                                                        const int32_t *__restrict__ seq_of_tile,
-                                                        const int32_t *__restrict__ seq_n,
-                                                        _Float16 *__restrict__ y, _Float16 *__restrict__ ylo) {
-  __shared__ __align__(16) float sP[4][16 * kPp];
-  __shared__ __align__(16) float sO[4][16 * kOp];
-  __shared__ float sML[4][16][2];
-  const int tile = blockIdx.x, h = blockIdx.y, z = blockIdx.z;
-  const int nsub = tile_n[tile] - 16 * z;  // rows of this 16-row half of the tile
-  if (nsub <= 0) return;                   // whole workgroup, before any barrier
-  const int row0 = tile_row0[tile] + 16 * z, pos0 = tile_pos0[tile] + 16 * z;
-  const int n = seq_n[seq_of_tile[tile]];
-  const int srow = row0 - pos0;
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, li = l & 15, kg = l >> 4;
+template <int QB>
+__global__ __launch_bounds__(256, 2) void laya_attn_kernel(const float *__restrict__ qkv, int d, int window, int ngroups,
+                                                           int per_head, const int32_t *__restrict__ grp_first,
+                                                           const int32_t *__restrict__ grp_count,
+                                                           const int32_t *__restrict__ tile_row0,
+                                                           const int32_t *__restrict__ tile_pos0,
+                                                           const int32_t *__restrict__ tile_n,
+                                                           const int32_t *__restrict__ tile_seq,
+                                                           const int32_t *__restrict__ seq_n, _Float16 *__restrict__ y,
+                                                           _Float16 *__restrict__ ylo) {
+  __shared__ __align__(16) f16x8 lds[2 * kKSlots + 2 * kVSlots];
+  f16x8 *const Kh = lds, *const Kl = Kh + kKSlots, *const Vh = Kl + kKSlots, *const Vl = Vh + kVSlots;
+  // workgroups go to the 8 XCDs round-robin; each XCD takes a contiguous range of (head, group) pairs, groups fastest, so
+  // the workgroups of one sequence and head read its rows through one L2
+  const int total = gridDim.x, xcd = blockIdx.x % 8, per = total / 8, rem = total % 8;
+  const int logical = xcd * per + min(xcd, rem) + blockIdx.x / 8;
+  const int h = logical / per_head, part = logical % per_head, grp = part % ngroups, z = part / ngroups;
+  const int t0 = grp_first[grp], cnt = grp_count[grp];
+  const int first = QB == 2 ? 0 : 2 * z, last = min(cnt, QB == 2 ? 4 : first + 2) - 1;
+  if (first >= cnt) return;  // whole workgroup, before any barrier
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, lr = l & 15, qg = l >> 4;
+  const int ti = QB == 2 ? w : first + w / 2, sub = QB == 2 ? 0 : 16 * (w & 1);
+  const int tile = t0 + min(ti, last);
+  const int nq = tile_n[tile] - sub;  // queries of this wave: rows sub .. sub + min(nq, 16 QB) of the tile
+  const bool active = ti <= last && nq > 0;
+  const int row0 = tile_row0[tile] + sub, pos0 = tile_pos0[tile] + sub;
+  const int n = seq_n[tile_seq[t0]];
   const int ld = 3 * d;
-  const float *kbase = qkv + int64_t(srow) * ld + d + h * kHD;  // key rows of the sequence
-  // Q operands: row li (rows past nsub repeat the last row and are never written)
-  half4v qh[4], ql[4];
-  {
-    const float *qr = qkv + int64_t(row0 + min(li, nsub - 1)) * ld + h * kHD;
+  const float *kbase = qkv + int64_t(tile_row0[t0] - tile_pos0[t0]) * ld + d + h * kHD;  // key rows of the sequence
+  const int plast = tile_pos0[t0 + last] + tile_n[t0 + last];
+  const int wlo = window < 0 ? 0 : max(0, tile_pos0[t0 + first] - window), whi = window < 0 ? n : min(n, plast + window);
+  const int kb1 = (whi + kKB - 1) / kKB;
+
+  f16x8 qh[QB][2], ql[QB][2];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) split_hl(*reinterpret_cast<const float4v *>(qr + 16 * g + 4 * kg), qh[g], ql[g]);
-  }
-  // visible keys of the 16 rows, in 16-key blocks split over the four waves
-  const int wlo = window < 0 ? 0 : max(0, pos0 - window);
-  const int whi = window < 0 ? n : min(n, pos0 + nsub + window);
-  const int b0 = wlo / 16, nb = (whi + 15) / 16 - b0;
-  const int bw0 = b0 + (nb * w) / 4, bw1 = b0 + (nb * (w + 1)) / 4;
-  float4v acc[4];
+  for (int qb = 0; qb < QB; ++qb) {
+    // rows past the tile repeat its last row and are never written
+    const float *qr = qkv + int64_t(row0 - sub + min(sub + qb * 16 + lr, sub + nq - 1)) * ld + h * kHD + 8 * qg;
 #pragma unroll
-  for (int b = 0; b < 4; ++b) acc[b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-  float m[4], lsum[4];
+    for (int c = 0; c < 2; ++c) {
+      float v[8];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    m[r] = -FLT_MAX;
-    lsum[r] = 0.0f;
-  }
-  float *myP = sP[w];
-  KVBlock cur, nxt;
-  if (bw0 < bw1) laya_load_kv(cur, kbase, ld, d, 16 * bw0, n, li, kg);
-  for (int bi = bw0; bi < bw1; ++bi) {
-    laya_load_kv(nxt, kbase, ld, d, 16 * min(bi + 1, bw1 - 1), n, li, kg);  // the last one reloads its own
-    float4v s = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      half4v kh, kl;
-      split_hl(cur.k[g], kh, kl);
-      s = mfma3(qh[g], ql[g], kh, kl, s);
+      for (int e = 0; e < 2; ++e) *reinterpret_cast<float4v *>(v + 4 * e) = *reinterpret_cast<const float4v *>(qr + 32 * c + 4 * e);
+      split8_pk(v, qh[qb][c], ql[qb][c]);
     }
-    const int key = 16 * bi + li;
-    float corr[4];
+  }
+  float4v acc[QB][4];
+  float m[QB], lsum[QB];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 4 * kg + r, qpos = pos0 + row;
-      const bool ok = row < nsub && key < n && (window < 0 || (key - qpos <= window && qpos - key <= window));
-      const float a = s[r] * kScoreLog2;  // q.k / sqrt(64) in base-2 units
-      const float mt = row_max16(ok ? a : -FLT_MAX);
-      const float mn = fmaxf(m[r], mt);
-      const float p = ok ? __builtin_amdgcn_exp2f(a - mn) : 0.0f;
-      const float ps = row_sum(p);
-      corr[r] = 1.0f;
-      if (mt > -FLT_MAX) {
-        corr[r] = m[r] == mn ? 1.0f : m[r] > -FLT_MAX ? __builtin_amdgcn_exp2f(m[r] - mn) : 0.0f;
-        lsum[r] = lsum[r] * corr[r] + ps;
-        m[r] = mn;
+  for (int qb = 0; qb < QB; ++qb) {
+#pragma unroll
+    for (int b = 0; b < 4; ++b) acc[qb][b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    m[qb] = -1e30f;  // finite: 2^(-inf - m) = 0 while no key of a window has been seen
+    lsum[qb] = 0.0f;
+  }
+  // this thread's part of a block: K chunks of rows tid / 8 and 32 + tid / 8, V of dim l, keys 16 w .. 16 w + 15 (key rows
+  // past the sequence repeat its last row and are masked)
+  float4v kf[2][2];
+  float vf[16];
+  auto load = [&](int kb) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float *kr = kbase + int64_t(min(kb * kKB + 32 * i + (tid >> 3), n - 1)) * ld + (tid & 7) * 8;
+      kf[i][0] = *reinterpret_cast<const float4v *>(kr);
+      kf[i][1] = *reinterpret_cast<const float4v *>(kr + 4);
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) vf[e] = kbase[int64_t(min(kb * kKB + 16 * w + e, n - 1)) * ld + d + l];
+  };
+  auto stage = [&] {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = kf[i][e / 4][e % 4];
+      const int row = 32 * i + (tid >> 3), slot = row * 8 + ((tid & 7) ^ laya_kswz(row));
+      split8_pk(v, Kh[slot], Kl[slot]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) split8_pk(vf + 8 * i, Vh[l * 9 + 2 * w + i], Vl[l * 9 + 2 * w + i]);
+  };
+  const int kr0 = 8 * (lr >> 2) + (lr & 3), ksw = laya_kswz(kr0);
+  load(wlo / kKB);
+  for (int kb = wlo / kKB; kb < kb1; ++kb) {
+    if (kb > wlo / kKB) __syncthreads();  // every wave is done with the previous block
+    stage();
+    __syncthreads();
+    if (kb + 1 < kb1) load(kb + 1);
+    const int k0 = kb * kKB;
+    // a block outside every window of the wave adds nothing
+    if (!active || (window >= 0 && (k0 + kKB - 1 < pos0 - window || k0 > pos0 + min(nq, 16 * QB) - 1 + window))) continue;
+    float4v s[QB][2][2];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[qb][i / 2][i % 2] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int ck = 0; ck < 2; ++ck)
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+          const int slot = (ck * 32 + kr0 + 4 * hh) * 8 + ((4 * c + qg) ^ ksw);
+          const f16x8 kh = Kh[slot], kl = Kl[slot];
+#pragma unroll
+          for (int qb = 0; qb < QB; ++qb) {
+            s[qb][ck][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[qb][c], s[qb][ck][hh], 0, 0, 0);
+            s[qb][ck][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[qb][c], s[qb][ck][hh], 0, 0, 0);
+            s[qb][ck][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[qb][c], s[qb][ck][hh], 0, 0, 0);
+          }
+        }
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[qb][i / 2][i % 2][e] *= kScoreLog2;
+    if (k0 + kKB > n || (window >= 0 && (k0 + kKB - 1 - pos0 > window || pos0 + 16 * QB - 1 - k0 > window))) {
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        const int qpos = pos0 + qb * 16 + lr;
+        const int hi = min(n - 1, window < 0 ? n - 1 : qpos + window) - k0 - 8 * qg;
+        const int lo = (window < 0 ? 0 : qpos - window) - k0 - 8 * qg;
+#pragma unroll
+        for (int ck = 0; ck < 2; ++ck)
+#pragma unroll
+          for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int j = ck * 32 + 4 * hh + e;
+              if (j > hi || j < lo) s[qb][ck][hh][e] = -INFINITY;
+            }
       }
-      myP[row * kPp + li] = p;
     }
-    if (__any(corr[0] != 1.0f || corr[1] != 1.0f || corr[2] != 1.0f || corr[3] != 1.0f)) {
 #pragma unroll
-      for (int b = 0; b < 4; ++b)
+    for (int qb = 0; qb < QB; ++qb) {
+      float mt = -INFINITY;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[b][r] *= corr[r];
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mt = fmaxf(mt, s[qb][i / 2][i % 2][e]);
+      mt = fmaxf(mt, __shfl_xor(mt, 16));
+      mt = fmaxf(mt, __shfl_xor(mt, 32));
+      // the exponent base moves only when a score exceeds it by more than 8; lanes that keep theirs multiply by exactly 1
+      const bool grow = mt > m[qb] + 8.0f;
+      if (__any(grow)) {
+        const float mn = grow ? mt : m[qb];
+        const float alpha = __builtin_amdgcn_exp2f(m[qb] - mn);
+        lsum[qb] *= alpha;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[qb][b][r] *= alpha;
+        m[qb] = mn;
+      }
+      float rs = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float p = __builtin_amdgcn_exp2f(s[qb][i / 2][i % 2][e] - m[qb]);
+          s[qb][i / 2][i % 2][e] = p;
+          rs += p;
+        }
+      rs += __shfl_xor(rs, 16);
+      rs += __shfl_xor(rs, 32);
+      lsum[qb] += rs;
     }
-    // P moves between the lanes of this wave through its own LDS rows: the wave barriers order the
-    // stores above before the read below, and this read before the next block's stores
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    half4v ph, pl;
-    split_hl(*reinterpret_cast<const float4v *>(myP + li * kPp + 4 * kg), ph, pl);
-    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int ck = 0; ck < 2; ++ck) {
+      f16x8 ph[QB], pl[QB];
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        float pv[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          pv[e] = s[qb][ck][0][e];
+          pv[4 + e] = s[qb][ck][1][e];
+        }
+        split8_pk(pv, ph[qb], pl[qb]);
+      }
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const int slot = (b * 16 + lr) * 9 + 4 * ck + qg;
+        const f16x8 vh = Vh[slot], vl = Vl[slot];
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+          acc[qb][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[qb], acc[qb][b], 0, 0, 0);
+          acc[qb][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[qb], acc[qb][b], 0, 0, 0);
+          acc[qb][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[qb], acc[qb][b], 0, 0, 0);
+        }
+      }
+    }
+  }
+  if (!active) return;
+  // acc[qb][b][r]: dim 16 b + 4 qg + r of query qb * 16 + lr
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    if (qb * 16 + lr >= nq) continue;
+    const float inv = 1.0f / lsum[qb];
+    const int64_t base = int64_t(row0 + qb * 16 + lr) * d + h * kHD + 4 * qg;
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      half4v vh, vl;
-      split_hl(float4v{cur.v[4 * b], cur.v[4 * b + 1], cur.v[4 * b + 2], cur.v[4 * b + 3]}, vh, vl);
-      acc[b] = mfma3(ph, pl, vh, vl, acc[b]);
+      typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+      half4v oh, ol;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        _Float16 hi, lo;
+        split_f16(acc[qb][b][j] * inv, hi, lo);
+        oh[j] = hi;
+        ol[j] = lo;
+      }
+      *reinterpret_cast<half4v *>(y + base + 16 * b) = oh;
+      if (ylo) *reinterpret_cast<half4v *>(ylo + base + 16 * b) = ol;
     }
-    cur = nxt;
-  }
-  // merge the four key ranges: O = sum_w e^(m_w - M) O_w / sum_w e^(m_w - M) l_w
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) sO[w][(4 * kg + r) * kOp + 16 * b + li] = acc[b][r];
-  if (li == 0)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      sML[w][4 * kg + r][0] = m[r];
-      sML[w][4 * kg + r][1] = lsum[r];
-    }
-  __syncthreads();
-  const int row = tid >> 4, d4 = (tid & 15) * 4;
-  if (row >= nsub) return;
-  float M = -FLT_MAX;
-#pragma unroll
-  for (int v = 0; v < 4; ++v)
-    if (sML[v][row][1] > 0.0f) M = fmaxf(M, sML[v][row][0]);
-  float L = 0.0f, o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    if (!(sML[v][row][1] > 0.0f)) continue;
-    const float f = __builtin_amdgcn_exp2f(sML[v][row][0] - M);
-    L += f * sML[v][row][1];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] += f * sO[v][row * kOp + d4 + e];
-  }
-  const float inv = 1.0f / L;
-  const int64_t base = int64_t(row0 + row) * d + h * kHD + d4;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    _Float16 hh, hl;
-    split_f16(o[e] * inv, hh, hl);
-    y[base + e] = hh;
-    if (ylo) ylo[base + e] = hl;
   }
 }
 
@@ -372,13 +426,17 @@ void launch_laya_rope(float *qkv, int T, int d, int hd, const float *cosT, const
 }
 
 void launch_laya_attn(const float *qkv, int d, int hd, int window, const int32_t *tile_row0, const int32_t *tile_pos0,
-                      const int32_t *tile_n, const int32_t *tile_seq, const int32_t *seq_n, int ntiles, _Float16 *y,
-                      _Float16 *ylo, hipStream_t st) {
+                      const int32_t *tile_n, const int32_t *tile_seq, const int32_t *seq_n, const int32_t *grp_first,
+                      const int32_t *grp_count, int ngroups, _Float16 *y, _Float16 *ylo, hipStream_t st) {
   LG_REQUIRE(hd == kHD, "laya attention: head_dim %d (kernel is built for 64)", hd);
-  LG_REQUIRE(ntiles > 0 && d % kHD == 0 && d >= kHD, "laya attention: bad shape");
-  // tiles hold at most 32 rows: two 16-row halves per tile (grid z)
-  hipLaunchKernelGGL(laya_attn_kernel, dim3(ntiles, d / kHD, 2), dim3(256), 0, st, qkv, d, window, tile_row0, tile_pos0,
-                     tile_n, tile_seq, seq_n, y, ylo);
+  LG_REQUIRE(ngroups > 0 && d % kHD == 0 && d >= kHD, "laya attention: bad shape");
+  const int heads = d / kHD;
+  const bool small = int64_t(ngroups) * heads < device_cus();
+  const int per_head = small ? 2 * ngroups : ngroups;
+  LG_REQUIRE(int64_t(per_head) * heads < (1ll << 31), "laya attention: too many tiles");
+  const auto fn = small ? laya_attn_kernel<1> : laya_attn_kernel<2>;
+  hipLaunchKernelGGL(fn, dim3(per_head * heads), dim3(256), 0, st, qkv, d, window, ngroups, per_head, grp_first, grp_count,
+                     tile_row0, tile_pos0, tile_n, tile_seq, seq_n, y, ylo);
   HIP_CHECK(hipGetLastError());
 }
 

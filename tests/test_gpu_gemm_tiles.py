@@ -40,7 +40,7 @@ def test_decoder_tilings_agree(lh, preset, precision, layers):
 def test_encoder_tilings_agree(lh):
     eng = lh.Engine(lh.Gguf.from_bytes(lh.SynthImage("laya-english", seed=31, n_layers=4)))
     rng = np.random.default_rng(9)
-    inputs = [(rng.integers(0, 1000, n).astype(np.int32), [0, n - 1], n % 3) for n in (2, 17, 32, 33, 65, 129, 300, 511)]
+    inputs = [(rng.integers(0, 1000, n).astype(np.int32), [0, n - 1], n % 3) for n in (2, 17, 32, 33, 63, 64, 65, 81, 129, 193, 300, 511)]
     whole = eng.laya_forward(inputs * 8)
     for i, x in enumerate(inputs):
         print(f"encoder {len(x[0])} tokens alone", flush=True)
