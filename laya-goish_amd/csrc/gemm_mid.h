@@ -6,7 +6,7 @@
 // stage through registers keep one K step in flight (the tiles of gemm_tiles.h: ~2 us a 128-deep step of 64 x 128 at 80
 // workgroups).  Here every operand byte moves by LDS-DMA (buffer_load ... lds) with no registers, no conversion, and
 // S stages of 64-deep steps: up to S - 1 steps are in flight while one is consumed.  Measured (chained launches): Q8_0 down
-// (2048 x 5632) at 301 rows 87 -> 45 us, Q6_K down (3584 x 18944) at 700 rows 768 -> 475 us, F16 512 x 512 at 144 rows 8.0 ->
+// (2048 x 5632) at 301 rows 87 -> 45 us, Q6_K down (3584 x 18944) at 700 rows 768 -> 385 us, F16 512 x 512 at 144 rows 8.0 ->
 // 3.8 us.  A step's time then follows the bytes that pass through the LDS (24 KB in, 48 KB out for 64 x 64), not the depth
 // of the pipeline: five stages of 64 x 64 take as long as three.
 //
@@ -15,6 +15,8 @@
 // slots, chunk c of row r at slot c ^ (r % 8): eight consecutive lanes of an operand read take the eight 16-byte
 // groups of 128 bytes, without bank conflicts.
 #pragma once
+#include <type_traits>
+
 #include "gemm_tiles.h"
 #include "gemm_wide.h"
 
@@ -65,9 +67,10 @@ struct Operands {
 // acc += the K loop over nk steps of 64.  aoff / boff: this lane's byte offsets of DMA instruction q of an A / W
 // plane (rows 32 q + 8 wave + lane / 8), soff: of the scale block, sstep its bytes per step.
 // Step k: the reads of its second 32-deep chunk issue before the MFMAs of the first; then (barrier) step k + 1 has
-// landed and every wave has read all of step k, so the DMA of step k + S goes into its stage and the reads of step k +
-// 1's first chunk issue before the MFMAs of the second.  No step past the last is fetched; once none is left to issue,
-// the wait is for all that is in flight.
+// landed and every wave has read all of step k, so the reads of step k + 1's first chunk issue, and the DMA of step k + S
+// into step k's stage goes with the MFMAs of the second chunk (ahead of the reads it held them back: Q6_K 3584 x 18944 at
+// 700 rows 473 -> 385 us, F16 1024 x 3584 at 1024 rows 24.3 -> 21.9).  No step past the last is fetched; once none is left
+// to issue, the wait is for all that is in flight.
 template <int NPB, bool SCALED, int HM, int HN, int S>
 __device__ __forceinline__ void k_loop(uint8_t *lds, f32x4 (&acc)[HM][HN], const Operands &o, const uint32_t (&aoff)[HM],
                                        const uint32_t (&boff)[HN], uint32_t soff, uint32_t sstep, int nk, int wave,
@@ -76,27 +79,29 @@ __device__ __forceinline__ void k_loop(uint8_t *lds, f32x4 (&acc)[HM][HN], const
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef __attribute__((address_space(3))) void *lds_ptr;
 #endif
-  auto issue = [&](int k, int st) {
+  // DMA instruction i of step k into stage st
+  auto dma = [&](int k, int st, int i) {
 #if defined(__HIP_DEVICE_COMPILE__)
     // device pass only: with a run-time voffset this builtin keeps the host pass from emitting the launch stub
     uint8_t *base = lds + st * G::kBytes + wave * 1024;
     const uint32_t kb = uint32_t(k) * ROWB;
-#pragma unroll
-    for (int q = 0; q < HM; ++q) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(o.ah, (lds_ptr)(base + q * 4096), 16, aoff[q], kb, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(o.al, (lds_ptr)(base + G::kALo + q * 4096), 16, aoff[q], kb, 0, 0);
-    }
-#pragma unroll
-    for (int q = 0; q < HN; ++q) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(o.bh, (lds_ptr)(base + G::kBHi + q * 4096), 16, boff[q], kb, 0, 0);
-      if constexpr (NPB == 2)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(o.bl, (lds_ptr)(base + G::kBLo + q * 4096), 16, boff[q], kb, 0, 0);
-    }
-    // every wave moves the scale block (the same bytes to the same place): one count of DMA for all waves
-    if constexpr (SCALED)
+    if (i < 2 * HM) {
+      const int q = i / 2;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(i % 2 ? o.al : o.ah, (lds_ptr)(base + (i % 2 ? G::kALo : 0) + q * 4096), 16,
+                                               aoff[q], kb, 0, 0);
+    } else if (i < 2 * HM + NPB * HN) {
+      const int q = (i - 2 * HM) / NPB, lo = (i - 2 * HM) % NPB;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(lo ? o.bl : o.bh, (lds_ptr)(base + (lo ? G::kBLo : G::kBHi) + q * 4096), 16,
+                                               boff[q], kb, 0, 0);
+    } else {  // every wave moves the scale block (the same bytes to the same place): one count of DMA for all waves
       __builtin_amdgcn_raw_ptr_buffer_load_lds(o.sc, (lds_ptr)(lds + st * G::kBytes + G::kScl), 16, soff,
                                                uint32_t(k) * sstep, 0, 0);
+    }
 #endif
+  };
+  auto issue = [&](int k, int st) {
+#pragma unroll
+    for (int i = 0; i < G::kDma; ++i) dma(k, st, i);
   };
   const int lr = lane & 15, g = lane >> 4, wm = wave >> 1, wn = wave & 1;
   const int arow = (wm * 16 * HM + lr) * ROWB, brow = (wn * 16 * HN + lr) * ROWB;
@@ -121,35 +126,47 @@ __device__ __forceinline__ void k_loop(uint8_t *lds, f32x4 (&acc)[HM][HN], const
         f.d[j] = *reinterpret_cast<const float *>(p + G::kScl + (ck * 32 * HN + wn * 16 * HN + j * 16 + lr) * 4);
     }
   };
-  auto compute = [&](const Frag &f) {
+  // The MFMAs of one 32-deep chunk; with DMA, the instructions of step dk into stage dst spread between them (a wave's
+  // next MFMA waits behind a DMA instruction that the texture unit has not taken yet).
+  constexpr int kMfma = HM * HN * (NPB == 2 ? 3 : 2);
+  auto compute = [&](const Frag &f, auto with_dma, int dk, int dst) {
     if constexpr (SCALED) {
+      // column j's MFMAs (hi then lo chains of its row blocks) issue between the scale FMAs of column j - 1
       const f32x4 zero = {};
+      f32x4 p[2][HM];
 #pragma unroll
-      for (int j = 0; j < HN; ++j) {
-        f32x4 p[HM];
+      for (int j = 0; j <= HN; ++j) {
+        if (j < HN) {
 #pragma unroll
-        for (int i = 0; i < HM; ++i) p[i] = MFMA(f.ah[i], f.b[j], zero);
+          for (int i = 0; i < HM; ++i) p[j & 1][i] = MFMA(f.ah[i], f.b[j], zero);
 #pragma unroll
-        for (int i = 0; i < HM; ++i) p[i] = MFMA(f.al[i], f.b[j], p[i]);
+          for (int i = 0; i < HM; ++i) p[j & 1][i] = MFMA(f.al[i], f.b[j], p[j & 1][i]);
+        }
+        if (j > 0) {
 #pragma unroll
-        for (int i = 0; i < HM; ++i)
+          for (int i = 0; i < HM; ++i)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i][j][r] += f.d[j] * p[i][r];
+            for (int r = 0; r < 4; ++r) acc[i][j - 1][r] += f.d[j - 1] * p[(j - 1) & 1][i][r];
+        }
+#pragma unroll
+        for (int q = 0; q < 2 * HM; ++q) {
+          if (j < HN) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA of column j
+          if (j > 0) __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);   // two FMAs of column j - 1
+        }
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < HN; ++j)
+      for (int n = 0; n < kMfma; ++n) {
+        const int pass = n / (HM * HN), j = n / HM % HN, i = n % HM;
+        acc[i][j] = MFMA(pass == 1 ? f.al[i] : f.ah[i], pass == 2 ? f.c[NPB == 2 ? j : 0] : f.b[j], acc[i][j]);
 #pragma unroll
-        for (int i = 0; i < HM; ++i) acc[i][j] = MFMA(f.ah[i], f.b[j], acc[i][j]);
-#pragma unroll
-      for (int j = 0; j < HN; ++j)
-#pragma unroll
-        for (int i = 0; i < HM; ++i) acc[i][j] = MFMA(f.al[i], f.b[j], acc[i][j]);
-      if constexpr (NPB == 2)
-#pragma unroll
-        for (int j = 0; j < HN; ++j)
-#pragma unroll
-          for (int i = 0; i < HM; ++i) acc[i][j] = MFMA(f.ah[i], f.c[j], acc[i][j]);
+        for (int q = 0; q < G::kDma; ++q)
+          if (decltype(with_dma)::value && q * kMfma / G::kDma == n) {
+            __builtin_amdgcn_sched_barrier(0);
+            dma(dk, dst, q);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+      }
     }
   };
 
@@ -165,18 +182,24 @@ __device__ __forceinline__ void k_loop(uint8_t *lds, f32x4 (&acc)[HM][HN], const
   for (int k = 0; k < nk; ++k) {
     read(st, 1, f1);
     __builtin_amdgcn_sched_barrier(0);  // the reads issue ahead of the MFMAs that cover them
-    compute(f0);
+    compute(f0, std::false_type{}, 0, 0);
     const int nst = st + 1 == S ? 0 : st + 1;
     if (k + 1 < nk) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave has read all of step k
       if (k + S - 1 < nk) wait_vm<(S - 2) * G::kDma>();
       else wait_vm<0>();
       bare_barrier();
-      if (k + S < nk) issue(k + S, st);
       read(nst, 0, f0);
       __builtin_amdgcn_sched_barrier(0);
     }
-    compute(f1);
+    if constexpr (SCALED) {  // spread among the scale FMAs the DMA cost 8-15%
+      if (k + S < nk) issue(k + S, st);
+      compute(f1, std::false_type{}, 0, 0);
+    } else if (k + S < nk) {
+      compute(f1, std::true_type{}, k + S, st);
+    } else {
+      compute(f1, std::false_type{}, 0, 0);
+    }
     st = nst;
   }
 }

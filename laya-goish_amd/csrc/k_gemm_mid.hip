@@ -15,29 +15,30 @@ using wide::WQ8;
 // Tile configurations: (HM, HN, stages).
 enum Tile { T11, T12, T22, T24, T24D, T44, kTiles, kNoTile = -1 };
 
-// Microseconds per 64-deep K step of one workgroup alone on a CU (one) and of two sharing it (two): (launch time -
-// 3 us) / (K / 64) over M 24-1437 and the q|k|v, o, gate|up and down shapes of the workload models (weights rotating
-// through 1.4 GB).  Two where the LDS holds a single workgroup is twice one.  0: not a configuration of the mode.
+// What a launch takes beyond ~3 us: microseconds per 64-deep K step of a workgroup alone on a CU (one) and of two sharing
+// it (two; 0: the LDS holds one), and a round's fill and drain.  Fitted to launches of M 24-1437 over the q|k|v, o, gate|up
+// and down shapes of the workload models (weights rotating through 1 GB).  one = 0: not a configuration of the mode.
 struct StepCost {
-  float one, two;
+  float one, two, fill;
 };
 constexpr StepCost kCost[4][kTiles] = {
-    /* WQ8 */ {{0.24f, 0.40f}, {0.31f, 0.54f}, {0.46f, 0.78f}, {0.84f, 1.03f}, {0.70f, 1.40f}, {1.11f, 2.25f}},
-    /* W1  */ {{0.20f, 0.36f}, {0.24f, 0.47f}, {0.36f, 0.70f}, {0.80f, 0.95f}, {0.57f, 1.14f}, {0.95f, 1.90f}},
-    /* W2  */ {{0.27f, 0.50f}, {0.43f, 0.86f}, {0.49f, 0.98f}, {0, 0}, {0.85f, 1.70f}, {1.50f, 3.00f}},
-    /* WQ4 */ {{0.24f, 0.40f}, {0.31f, 0.54f}, {0.46f, 0.78f}, {0, 0}, {0.70f, 1.40f}, {1.11f, 2.25f}},
+    /* WQ8 */ {{0.23f, 0.40f, 1}, {0.30f, 0.54f, 1}, {0.46f, 0.78f, 1}, {0.84f, 1.03f, 1}, {0.68f, 0, 1}, {1.14f, 0, 1}},
+    /* W1  */ {{0.19f, 0.36f, 0.5f}, {0.23f, 0.46f, 1}, {0.27f, 0.68f, 2}, {0.78f, 0.90f, 2}, {0.41f, 0, 2}, {0.66f, 0, 6.5f}},
+    /* W2  */ {{0.26f, 0.50f, 1}, {0.43f, 0.74f, 1}, {0.44f, 0, 2}, {0, 0, 0}, {0.73f, 0, 2}, {1.29f, 0, 6}},
+    /* WQ4 */ {{0.24f, 0.40f, 1}, {0.31f, 0.54f, 1}, {0.46f, 0.78f, 2}, {0, 0, 0}, {0.70f, 0, 2}, {1.14f, 0, 3}},
 };
 constexpr int kHM[kTiles] = {1, 1, 2, 2, 2, 4}, kHN[kTiles] = {1, 2, 2, 4, 4, 4};
 // a 256 x 256 tile's microseconds per 64-deep step, one workgroup per CU (mode order as above; F16 at 168 and 198 tiles
 // of K 1024, the others from full rounds)
 constexpr float kWideStep[4] = {3.5f, 2.75f, 4.7f, 3.5f};
 
-// Microseconds of `nk` steps: rounds of two workgroups per CU, the last one alone when half a round or less is left, each
-// with the fill and drain of its pipeline.
-constexpr float kRound = 2.0f;
+// Microseconds of `nk` steps over rounds of two workgroups per CU (the last round alone when half of it or less is left), or
+// of one.
 float cost(const StepCost &c, int64_t tiles, int nk) {
-  const int64_t n = device_cus(), rounds = tiles / (2 * n), rest = tiles - rounds * 2 * n;
-  return float(rounds) * (c.two * nk + kRound) + (rest == 0 ? 0.0f : (rest <= n ? c.one : c.two) * nk + kRound);
+  const int64_t n = device_cus();
+  if (c.two == 0) return float((tiles + n - 1) / n) * (c.one * nk + c.fill);
+  const int64_t rounds = tiles / (2 * n), rest = tiles - rounds * 2 * n;
+  return float(rounds) * (c.two * nk + c.fill) + (rest == 0 ? 0.0f : (rest <= n ? c.one : c.two) * nk + c.fill);
 }
 
 // The cheapest configuration for M rows of a matrix of `rows` weight rows (only those of 64 columns when rope), and
@@ -136,7 +137,7 @@ void launch_tile(int tile, const Launch &l) {
       if constexpr (!kRope) launch_rows<EPI, MODE, 2, 4, w2 ? 3 : 4>(l);
       break;
     case T44:
-      if constexpr (!kRope) launch_rows<EPI, MODE, 4, 4, 2>(l);
+      if constexpr (!kRope) launch_rows<EPI, MODE, 4, 4, w2 ? 2 : 3>(l);
       break;
   }
 }
@@ -161,8 +162,11 @@ bool gemm_mid_ahead(int M, const DevMatrix &W, bool glu, int64_t wide_tiles) {
   const int mode = mid_mode(M, W);
   float c = 0.0f;
   if (mode < 0 || best_tile(mode, M, W, glu, false, &c) == kNoTile) return false;
+  // the costs are those of short launches; over more than two rounds of 256 x 256 tiles the card holds its power and the
+  // larger tiles, with fewer instructions an MFMA, win whatever their last round (the 16-request Q4_K/Q6_K
+  // batch, 3.5 rounds of Q6_K down: 31.4 against 34.0 ms), and below that they are given a seventh
   const int64_t rounds = (wide_tiles + device_cus() - 1) / device_cus();
-  return c < float(rounds) * (kWideStep[mode] * (W.cols / mid::BK) + kRound);
+  return rounds <= 2 && c * 1.15f < float(rounds) * (kWideStep[mode] * (W.cols / mid::BK) + 1.0f);
 }
 
 bool launch_gemm_mid(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi, float *C,
