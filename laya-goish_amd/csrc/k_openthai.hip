@@ -662,20 +662,16 @@ __global__ __launch_bounds__(256, 1) void ot_attn_kernel(const float *__restrict
     }
 }
 
-// ---------------------------------------------------------------- full attention on f32 MFMA
-// The same attention as ot_attn_kernel on v_mfma_f32_16x16x4_f32 (f32 operands, f32
-// accumulation), split over keys for parallelism.  Work item = (16 query rows of one sequence,
-// a range of <= 256 keys, 4 query heads sharing one KV head): one wave per query head.
-//   S = Q K^T: lane (i = l%16, kg = l/16) supplies Q[i][16g + 4kg + c] at step 4g + c: the
-//   contraction order over the 256 dims is a permutation, applied to K alike, so each operand
-//   is one float4 LDS read per 4 MFMAs.
-//   D layout: lane l holds S[4(l/16) + r][16 blk + l%16], r < 4.
-//   Online softmax per row (16-lane DPP row reductions); P goes through LDS to the A layout.
-//   O += P V over keys 16u + 4kg + c (V transposed in LDS, so again one float4 per 4 MFMAs).
-// Partial (m, l, O) per item and head; ot_attn_combine_kernel merges an item's key ranges.
+// ---------------------------------------------------------------- full attention on MFMA
+// The same attention as ot_attn_kernel, split over keys for parallelism.  Work item = (16 query rows of one sequence, a
+// range of <= 256 keys, 4 query heads sharing one KV head): one wave per query head.  Scores and output are taken
+// transposed (keys, then dims, as rows; queries as columns), so a lane's probabilities are already the operand of
+// its output product: no P tile in LDS, two lane swaps a softmax reduction, and 75 KB of LDS and 247 registers leave room
+// for two workgroups a CU, one computing while the other waits for its tile (with P through LDS, row reductions of four
+// rows a lane and one workgroup a CU: 1437 tokens, 8 heads, 103 us a layer against 69).
+// Partial (m, l, O) per item and head, m in base-2 units; ot_attn_combine_kernel merges an item's key ranges.
 constexpr int kQT = 16;    // query rows per item
 constexpr int kKC = 256;   // keys per item
-constexpr int kPp = 36;    // padded row of the P tile [16 rows][32 keys]
 
 // One 32-key tile of K rows and V rows (from the projection) for 256 threads, 8 float4 each; keys past khi
 // are clamped to khi - 1 (masked by the caller).  K: kr[2 j + u] holds dims 8 o + 4 u .. + 3 of key i, with
@@ -703,13 +699,13 @@ __device__ __forceinline__ void ot_load_kv(float4v (&kr)[8], float4v (&vr)[8], c
 
 // The products on v_mfma_f32_16x16x32_f16 with every f32 operand split into f16 hi + lo (hi = f16(x),
 // lo = f16(x - hi)) and three products per pair (lo.hi, hi.lo, hi.hi; ~22 significant bits, f32
-// accumulation): Q split once into registers, each K and V tile split as it is staged, P as it is read
-// back.  LDS (dynamic): K hi and lo [32 keys][kKh], the transposed V tile hi and lo [256 dims][kVh], and each
-// wave's f32 P tile [16 rows][kPp].
+// accumulation): Q split once into registers, each K and V tile split as it is staged, P in registers.  LDS (dynamic): K hi
+// and lo [32 keys][kKh], the transposed V tile hi and lo [256 dims][kVh].
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
+constexpr float kOtScoreLog2 = 1.44269504088896341f / 16.0f;  // scores / sqrt(256) in base-2 units
 constexpr int kKh = kHD + 8;  // halves a staged K row (16 bytes of padding)
 constexpr int kVh = kAT + 8;  // halves a staged V^T row
-constexpr int kAttnLdsBytes = 2 * (2 * kAT * kKh + 2 * kHD * kVh) + 4 * 4 * kQT * kPp;
+constexpr int kAttnLdsBytes = 2 * (2 * kAT * kKh + 2 * kHD * kVh);  // two workgroups a CU
 
 __device__ __forceinline__ void split8(float4v a, float4v b, half8v &hi, half8v &lo) {
 #pragma unroll
@@ -730,7 +726,7 @@ __device__ __forceinline__ float4v mfma3h(half8v ah, half8v al, half8v bh, half8
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh, acc, 0, 0, 0);
 }
 
-__global__ __launch_bounds__(256, 1) void ot_attn_part_kernel(
+__global__ __launch_bounds__(256, 2) void ot_attn_part_kernel(
     const float *__restrict__ Qb, const float *__restrict__ Kb, const float *__restrict__ proj, int ldp, int hq,
     int hkv, const int32_t *__restrict__ it_row0, const int32_t *__restrict__ it_pos0,
     const int32_t *__restrict__ it_nq, const int32_t *__restrict__ it_klo, const int32_t *__restrict__ it_khi,
@@ -738,7 +734,6 @@ __global__ __launch_bounds__(256, 1) void ot_attn_part_kernel(
   extern __shared__ float4v attn_smem[];
   _Float16 *sKh = reinterpret_cast<_Float16 *>(attn_smem), *sKl = sKh + kAT * kKh;
   _Float16 *sVh = sKl + kAT * kKh, *sVl = sVh + kHD * kVh;
-  float *sP = reinterpret_cast<float *>(sVl + kHD * kVh);  // [4 waves][16 rows][kPp]
   const int item = blockIdx.x;
   const int row0 = it_row0[item], pos0 = it_pos0[item], nq = it_nq[item];
   const int klo = it_klo[item], khi = it_khi[item];
@@ -748,7 +743,7 @@ __global__ __launch_bounds__(256, 1) void ot_attn_part_kernel(
   const int kh = (blockIdx.y * 4) / (hq / hkv);
   const int qw = hq * kHD, kvw = hkv * kHD;
   const int li = l & 15, kg = l >> 4;
-  // this wave's Q rows as A operands: row li (rows past nq repeat row nq - 1 and are never written out),
+  // this wave's Q rows as B operands: row li (rows past nq repeat row nq - 1 and are never written out),
   // dims 32 s + 8 kg .. + 7 of k-step s
   half8v qh[8], ql[8];
   {
@@ -761,16 +756,10 @@ __global__ __launch_bounds__(256, 1) void ot_attn_part_kernel(
   float4v acc_o[16];
 #pragma unroll
   for (int b = 0; b < 16; ++b) acc_o[b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-  float m[4], lsum[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    m[r] = -FLT_MAX;
-    lsum[r] = 0.0f;
-  }
+  float m = -1e30f, lsum = 0.0f;  // of query li, in every lane that holds it; m finite before its first key
   const int kt0 = klo / kAT, kt1 = (khi + kAT - 1) / kAT;
   float4v kr[8], vr[8];
   ot_load_kv(kr, vr, Kb, proj, ldp, kvw, 2 * qw + kvw + kh * kHD, kh * kHD, srow, kt0, khi, tid);
-  float *myP = sP + w * (kQT * kPp);
   for (int kt = kt0; kt < kt1; ++kt) {
     __syncthreads();  // previous tile's readers are done
 #pragma unroll
@@ -778,8 +767,10 @@ __global__ __launch_bounds__(256, 1) void ot_attn_part_kernel(
       const int e = tid + 256 * j, i = e >> 5, o = e & 31;
       half8v h8, l8;
       split8(kr[2 * j], kr[2 * j + 1], h8, l8);
-      *reinterpret_cast<half8v *>(sKh + i * kKh + 8 * o) = h8;
-      *reinterpret_cast<half8v *>(sKl + i * kKh + 8 * o) = l8;
+      // key 8 a + 4 hh + b at row 16 hh + 4 a + b: a block's 16 rows are consecutive, without bank conflicts
+      const int row = ((i >> 2) & 1) * 16 + (i >> 3) * 4 + (i & 3);
+      *reinterpret_cast<half8v *>(sKh + row * kKh + 8 * o) = h8;
+      *reinterpret_cast<half8v *>(sKl + row * kKh + 8 * o) = l8;
     }
     {
       const int oc = tid >> 6, c4 = tid & 63;
@@ -800,57 +791,62 @@ __global__ __launch_bounds__(256, 1) void ot_attn_part_kernel(
     __syncthreads();
     // next tile's loads, unconditional (the last iteration reloads its own tile)
     ot_load_kv(kr, vr, Kb, proj, ldp, kvw, 2 * qw + kvw + kh * kHD, kh * kHD, srow, min(kt + 1, kt1 - 1), khi, tid);
-    // S = Q K^T, two 16x16 blocks of keys: B = K[16 kb + li][32 s + 8 kg .. + 7]
+    // S^T = K Q^T, two 16 x 16 blocks: row li of block hh is key 8 (li / 4) + 4 hh + li % 4, so lane l receives, for query
+    // li, keys 8 kg + 4 hh + 0..3: both blocks together are the eight keys of its P^T operand
     float4v s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int st = 0; st < 8; ++st) {
       const int o0 = li * kKh + 32 * st + 8 * kg, o1 = (16 + li) * kKh + 32 * st + 8 * kg;
-      s0 = mfma3h(qh[st], ql[st], *reinterpret_cast<const half8v *>(sKh + o0), *reinterpret_cast<const half8v *>(sKl + o0),
+      s0 = mfma3h(*reinterpret_cast<const half8v *>(sKh + o0), *reinterpret_cast<const half8v *>(sKl + o0), qh[st], ql[st],
                   s0);
-      s1 = mfma3h(qh[st], ql[st], *reinterpret_cast<const half8v *>(sKh + o1), *reinterpret_cast<const half8v *>(sKl + o1),
+      s1 = mfma3h(*reinterpret_cast<const half8v *>(sKh + o1), *reinterpret_cast<const half8v *>(sKl + o1), qh[st], ql[st],
                   s1);
     }
-    // scale, mask, online softmax; lane holds rows 4 kg + r, keys li and 16 + li
-    const int key0 = kt * kAT + li, key1 = key0 + 16;
-    float corr[4];
+    // scale to base 2, mask, online softmax
+    float p[8];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 4 * kg + r, qpos = pos0 + row;
-      const bool ok0 = key0 >= klo && key0 < khi && key0 <= qpos && row < nq;
-      const bool ok1 = key1 >= klo && key1 < khi && key1 <= qpos && row < nq;
-      const float a = s0[r] / 16.0f, b = s1[r] / 16.0f;
-      float mt = fmaxf(ok0 ? a : -FLT_MAX, ok1 ? b : -FLT_MAX);
-      mt = row_max16(mt);
-      const float mn = fmaxf(m[r], mt);
-      const bool any = mt > -FLT_MAX;
-      const float p0 = ok0 ? expf(a - mn) : 0.0f, p1 = ok1 ? expf(b - mn) : 0.0f;
-      const float ps = row_sum(p0 + p1);
-      corr[r] = 1.0f;
-      if (any) {
-        corr[r] = m[r] > -FLT_MAX ? expf(m[r] - mn) : 0.0f;
-        lsum[r] = lsum[r] * corr[r] + ps;
-        m[r] = mn;
-      }
-      myP[row * kPp + li] = p0;
-      myP[row * kPp + 16 + li] = p1;
+    for (int e = 0; e < 4; ++e) {
+      p[e] = s0[e] * kOtScoreLog2;
+      p[4 + e] = s1[e] * kOtScoreLog2;
     }
-    // rescale the running output only when some row's maximum moved (a wave-uniform branch:
-    // the accumulators stay in place otherwise)
-    if (__any(corr[0] != 1.0f || corr[1] != 1.0f || corr[2] != 1.0f || corr[3] != 1.0f)) {
+    const int last = min(khi - 1, pos0 + li) - kt * kAT - 8 * kg;  // keys past it are masked
+    float mt = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if (e > last) p[e] = -INFINITY;
+      mt = fmaxf(mt, p[e]);
+    }
+    mt = fmaxf(mt, __shfl_xor(mt, 16));
+    mt = fmaxf(mt, __shfl_xor(mt, 32));
+    // the exponent base moves only when a score exceeds it by more than 8; lanes that keep theirs multiply by exactly 1
+    const bool grow = mt > m + 8.0f;
+    if (__any(grow)) {
+      const float mn = grow ? mt : m;
+      const float alpha = __builtin_amdgcn_exp2f(m - mn);
+      lsum *= alpha;
 #pragma unroll
       for (int b = 0; b < 16; ++b)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc_o[b][r] *= corr[r];
+        for (int r = 0; r < 4; ++r) acc_o[b][r] *= alpha;
+      m = mn;
     }
-    // O += P V over the tile's 32 keys in one k-step: A = P[li][8 kg .. + 7], B = V[8 kg .. + 7][16 b + li]
+    float rs = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      p[e] = __builtin_amdgcn_exp2f(p[e] - m);
+      rs += p[e];
+    }
+    rs += __shfl_xor(rs, 16);
+    rs += __shfl_xor(rs, 32);
+    lsum += rs;
+    // O^T += V^T P^T over the tile's 32 keys in one k-step: A = V^T[16 b + li][8 kg .. + 7]
     {
       half8v ph, pl;
-      split8(*reinterpret_cast<const float4v *>(myP + li * kPp + 8 * kg),
-             *reinterpret_cast<const float4v *>(myP + li * kPp + 8 * kg + 4), ph, pl);
+      split8(float4v{p[0], p[1], p[2], p[3]}, float4v{p[4], p[5], p[6], p[7]}, ph, pl);
 #pragma unroll
       for (int b = 0; b < 16; ++b) {
         const int o = (16 * b + li) * kVh + 8 * kg;
-        acc_o[b] = mfma3h(ph, pl, *reinterpret_cast<const half8v *>(sVh + o), *reinterpret_cast<const half8v *>(sVl + o),
+        acc_o[b] = mfma3h(*reinterpret_cast<const half8v *>(sVh + o), *reinterpret_cast<const half8v *>(sVl + o), ph, pl,
                           acc_o[b]);
       }
     }
@@ -858,19 +854,12 @@ __global__ __launch_bounds__(256, 1) void ot_attn_part_kernel(
   // partial: [item][head][16 rows][256] O, then [item][head][16][2] (m, l)
   float *po = part + (int64_t(item) * hq + h) * (kQT * kHD + 2 * kQT);
 #pragma unroll
-  for (int b = 0; b < 16; ++b)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) po[(4 * kg + r) * kHD + 16 * b + li] = acc_o[b][r];
-  if (li == 0)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      po[kQT * kHD + 2 * (4 * kg + r)] = m[r];
-      po[kQT * kHD + 2 * (4 * kg + r) + 1] = lsum[r];
-    }
+  for (int b = 0; b < 16; ++b) *reinterpret_cast<float4v *>(po + li * kHD + 16 * b + 4 * kg) = acc_o[b];
+  if (kg == 0) *reinterpret_cast<float2 *>(po + kQT * kHD + 2 * li) = make_float2(m, lsum);
 }
 
-// Merge the key-range partials of one 16-row query tile and head: O = sum_s e^(m_s - M) O_s /
-// sum_s e^(m_s - M) l_s, then * sigmoid(gate) -> f16 planes.  256 threads: 16 rows x 16 dims
+// Merge the key-range partials of one 16-row query tile and head: O = sum_s 2^(m_s - M) O_s /
+// sum_s 2^(m_s - M) l_s, then * sigmoid(gate) -> f16 planes.  256 threads: 16 rows x 16 dims
 // groups of 16.
 __global__ __launch_bounds__(256) void ot_attn_combine_kernel(const float *__restrict__ part, const float *__restrict__ proj,
                                                               int ldp, int hq, const int32_t *__restrict__ cb_row0,
@@ -914,7 +903,7 @@ __global__ __launch_bounds__(256) void ot_attn_combine_kernel(const float *__res
 #pragma unroll
     for (int u = 0; u < G; ++u) {
       if (!(s0 + u < ns && ml[u].y > 0.0f)) continue;
-      const float f = expf(ml[u].x - M);
+      const float f = __builtin_amdgcn_exp2f(ml[u].x - M);  // m is in base-2 units
       L += f * ml[u].y;
 #pragma unroll
       for (int e = 0; e < 4; ++e)
