@@ -1209,7 +1209,7 @@ void Engine::decode_run(Seq &s, int32_t first, int steps, int32_t *tokens, float
       }
       gemv(x, head_, Epi::F32, lg, nullptr, final_norm_);
       prof.begin("argmax", stream);
-      if (i + 1 < steps) launch_argmax_embed(lg, V, tok + i + 1, emb_, emb_kind, d, x, stream);
+      if (i + 1 < steps) launch_argmax_embed(lg, V, tok + i + 1, emb_, emb_kind, d, x, part_v, part_i, stream);
       else launch_argmax(lg, V, tok + i + 1, part_v, part_i, stream);
       prof.end(double(V) * 4, 0, stream);
       if (logits) HIP_CHECK(hipMemcpyAsync(logits + size_t(i) * V, lg, size_t(V) * 4, hipMemcpyDeviceToHost, stream));

@@ -493,6 +493,100 @@ __device__ __forceinline__ void better(float &bv, int &bi, float v, int i) {
   }
 }
 
+// Two launches for long vectors (a single workgroup reads the 608 KB of a 152,064-entry vocabulary in 15.2 us, limited by what
+// one CU can load; the two together take 9.4): kArgParts workgroups each take a range, the last one merges.  At 32,000
+// entries the single launch below is ahead (5.7 us against 8.4).
+constexpr int kArgParts = 64;
+__global__ __launch_bounds__(kT) void argmax_part_kernel(const float *__restrict__ v, int n, float *__restrict__ part_v,
+                                                         int32_t *__restrict__ part_i) {
+  __shared__ float sv[kT / 64];
+  __shared__ int si[kT / 64];
+  const int per = ((n + kArgParts - 1) / kArgParts + 3) & ~3, lo = min(int(blockIdx.x) * per, n), hi = min(lo + per, n);
+  const int t = threadIdx.x, lane = t & 63;
+  float bv = -INFINITY;
+  int bi = -1;
+  constexpr int U = 4;
+  for (int k0 = lo + 4 * t; k0 < hi; k0 += 4 * kT * U) {
+    float w[U][4];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[u][e] = v[min(k0 + 4 * kT * u + e, n - 1)];  // all loads before any compare
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (k0 + 4 * kT * u + e < hi) better(bv, bi, w[u][e], k0 + 4 * kT * u + e);
+  }
+  auto merge = [&](float ov, int oi) {
+    if (oi >= 0 && (bi < 0 || ov > bv || (ov == bv && oi < bi))) {
+      bv = ov;
+      bi = oi;
+    }
+  };
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) merge(__shfl_xor(bv, m), __shfl_xor(bi, m));
+  if (lane == 0) {
+    sv[t >> 6] = bv;
+    si[t >> 6] = bi;
+  }
+  __syncthreads();
+  if (t == 0) {
+#pragma unroll
+    for (int w = 1; w < kT / 64; ++w) merge(sv[w], si[w]);
+    part_v[blockIdx.x] = bv;
+    part_i[blockIdx.x] = bi;
+  }
+}
+
+// The token's embedding row (ids clamped as embed_kernel clamps them) to x, four loads of a thread in flight.
+template <int THREADS>
+__device__ __forceinline__ void token_row(int tok, int n, const void *__restrict__ table, uint32_t kind, int d,
+                                          float *__restrict__ x) {
+  const int64_t row = int64_t(min(max(tok, 0), n - 1)) * d;
+  for (int k0 = threadIdx.x; k0 < d; k0 += 4 * THREADS) {
+    float w[4];
+    if (kind == LG_F16) {
+      uint16_t b[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) b[u] = static_cast<const uint16_t *>(table)[row + min(k0 + u * THREADS, d - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = half_bits(b[u]);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = static_cast<const float *>(table)[row + min(k0 + u * THREADS, d - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (k0 + u * THREADS < d) x[k0 + u * THREADS] = w[u];
+  }
+}
+
+// Merges the parts; with x, also writes the token's embedding row, as argmax_one<true>.
+__global__ __launch_bounds__(1024) void argmax_merge_kernel(const float *__restrict__ part_v, const int32_t *__restrict__ part_i,
+                                                          int n, int32_t *__restrict__ out, const void *__restrict__ table,
+                                                          uint32_t kind, int d, float *__restrict__ x) {
+  static_assert(kArgParts == 64, "one part a lane");
+  const int t = threadIdx.x, lane = t & 63;
+  float bv = part_v[lane];
+  int bi = part_i[lane];
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {  // every wave merges for itself
+    const float ov = __shfl_xor(bv, m);
+    const int oi = __shfl_xor(bi, m);
+    if (oi >= 0 && (bi < 0 || ov > bv || (ov == bv && oi < bi))) {
+      bv = ov;
+      bi = oi;
+    }
+  }
+  const int tok = bi >= 0 && bv > -INFINITY && bv < INFINITY ? bi : -1;  // -1: no finite maximum
+  if (t == 0) out[0] = tok;
+  if (x) token_row<1024>(tok, n, table, kind, d, x);
+}
+
+// from this length two launches
+constexpr int kArgLong = 65536;
+
 // One workgroup of 1024 threads over the whole vector (one launch: a decode step's argmax sits between
 // two dependent launches).  Thread t takes float4 words t, t + 1024, ... (their elements in index
 // order, so the strict `better` keeps the first of equal values), then the merge rule of the two-stage
@@ -554,10 +648,7 @@ __global__ __launch_bounds__(1024) void argmax_one(const float *__restrict__ v, 
   }
   if constexpr (EMB) {
     __syncthreads();
-    const int64_t row = int64_t(min(max(stok, 0), n - 1)) * d;
-    for (int k = t; k < d; k += 1024)
-      x[k] = kind == LG_F16 ? half_bits(static_cast<const uint16_t *>(table)[row + k])
-                            : static_cast<const float *>(table)[row + k];
+    token_row<1024>(stok, n, table, kind, d, x);
   }
 }
 
@@ -648,20 +739,28 @@ void launch_option_scores(const float *logits, int R, int k, float temperature, 
   HIP_CHECK(hipGetLastError());
 }
 
+static void launch_argmax_long(const float *logits, int V, int32_t *out, float *part_v, int32_t *part_i, const void *table,
+                               uint32_t kind, int d, float *x, hipStream_t st) {
+  LG_REQUIRE(part_v && part_i, "argmax: missing partials");
+  hipLaunchKernelGGL(argmax_part_kernel, dim3(kArgParts), dim3(kT), 0, st, logits, V, part_v, part_i);
+  hipLaunchKernelGGL(argmax_merge_kernel, dim3(1), dim3(1024), 0, st, part_v, part_i, V, out, table, kind, d, x);
+  HIP_CHECK(hipGetLastError());
+}
+
 void launch_argmax(const float *logits, int V, int32_t *out, float *part_v, int32_t *part_i,
                    hipStream_t st) {
   LG_REQUIRE(V > 0, "argmax: empty");
-  (void)part_v;  // the single-workgroup form needs no partials
-  (void)part_i;
+  if (V >= kArgLong) return launch_argmax_long(logits, V, out, part_v, part_i, nullptr, 0, 0, nullptr, st);
   hipLaunchKernelGGL(argmax_one<false>, dim3(1), dim3(1024), 0, st, logits, V, out, static_cast<const void *>(nullptr),
                      0u, 0, static_cast<float *>(nullptr));
   HIP_CHECK(hipGetLastError());
 }
 
 void launch_argmax_embed(const float *logits, int V, int32_t *out, const void *table, uint32_t kind, int d, float *x,
-                         hipStream_t st) {
+                         float *part_v, int32_t *part_i, hipStream_t st) {
   LG_REQUIRE(V > 0 && d > 0 && table && x, "argmax: bad arguments");
   LG_REQUIRE(kind == LG_F16 || kind == LG_F32, "embed: table must be F16/F32");
+  if (V >= kArgLong) return launch_argmax_long(logits, V, out, part_v, part_i, table, kind, d, x, st);
   hipLaunchKernelGGL(argmax_one<true>, dim3(1), dim3(1024), 0, st, logits, V, out, table, kind, d, x);
   HIP_CHECK(hipGetLastError());
 }

@@ -48,3 +48,27 @@ def test_encoder_tilings_agree(lh):
         assert_bits_equal(np.asarray(logits), np.asarray(whole[i][0]))
         assert_bits_equal(np.asarray(act), np.asarray(whole[i][1]))
     eng.close()
+
+
+def test_long_vocabulary_argmax(lh):
+    """Vocabularies of 65,536 entries and more take the argmax in two launches: each decoded token is the first
+    maximum of its step's logits, and the next step continues from it (a run equals single steps)."""
+    eng = lh.Engine(lh.Gguf.from_bytes(lh.SynthImage("q4km-7b", seed=3, n_layers=1)), kv_tokens=4096)
+    ids = np.random.default_rng(3).integers(0, 1000, 70).astype(np.int32)
+    runs = []
+    for single in (False, True):
+        s = eng.seq_create()
+        eng.forward(s, ids, [len(ids) - 1], vocab_ids=[0])
+        if single:
+            tok, toks = 5, []
+            for _ in range(6):
+                t, logits = eng.decode(s, tok, 1, want_logits=True)
+                tok = int(t[-1])
+                assert tok == int(np.argmax(logits[0]))
+                toks.append(tok)
+            runs.append(toks)
+        else:
+            runs.append([int(t) for t in eng.decode(s, 5, 6)])
+        eng.seq_free(s)
+    assert runs[0] == runs[1]
+    eng.close()
