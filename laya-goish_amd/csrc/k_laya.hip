@@ -21,9 +21,7 @@ __device__ float block_sum_ln(float v, float *red) {
   v = wave_sum_dpp(v);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  const float s = (red[0] + red[1]) + (red[2] + red[3]);
-  __syncthreads();
-  return s;
+  return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 __device__ __forceinline__ float gelu_tanh_f(float x) {
@@ -34,48 +32,53 @@ __device__ __forceinline__ float gelu_tanh_f(float x) {
 // row read once into registers (d <= 4096, d % 4 == 0).  Row r of the output reads input row
 // rows[r] (rows == nullptr: r).  Output: f16 hi/lo planes (y16, y16lo) or f32 (y32).  The add
 // row (f32 [3][d]) is add + sel[seq[r]] * d.
+template <int NI>
 __global__ __launch_bounds__(kT) void layer_norm_kernel(const float *__restrict__ x, const int32_t *__restrict__ rows,
                                                         int d, const float *__restrict__ w, const float *__restrict__ b,
                                                         float eps, const float *__restrict__ add,
                                                         const int32_t *__restrict__ seq, const int32_t *__restrict__ sel,
                                                         _Float16 *__restrict__ y16, _Float16 *__restrict__ y16lo,
                                                         float *__restrict__ y32) {
-  __shared__ float red[4];
+  __shared__ float red[8];
   const int r = blockIdx.x;
   const float4 *row = reinterpret_cast<const float4 *>(x + int64_t(rows ? rows[r] : r) * d);
   const int n4 = d >> 2;
-  float4 v[4];
+  const float *addrow = add ? add + int64_t(sel[seq[r]]) * d : nullptr;
+  // the row, its weights, biases and added row in one round trip (clamped indices: no load waits for a sum), 16 bytes each
+  // (weights after the two sums: 31,488 rows of 768 37.9 us against 34.4, 45 rows 3.5 against 3.2)
+  float4 v[NI], wr[NI], br[NI], ar[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int k = min(int(threadIdx.x) + i * kT, n4 - 1);
+    v[i] = row[k];
+    wr[i] = w ? reinterpret_cast<const float4 *>(w)[k] : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+    br[i] = b ? reinterpret_cast<const float4 *>(b)[k] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    ar[i] = addrow ? reinterpret_cast<const float4 *>(addrow)[k] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
   float s = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int k = threadIdx.x + i * kT;
-    v[i] = k < n4 ? row[k] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
-  }
+  for (int i = 0; i < NI; ++i)
+    if (int(threadIdx.x) + i * kT < n4) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
   const float mean = block_sum_ln(s, red) / float(d);
   float q = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < NI; ++i) {
     const int k = threadIdx.x + i * kT;
     if (k < n4) {
       const float a = v[i].x - mean, bb = v[i].y - mean, c = v[i].z - mean, e = v[i].w - mean;
       q += (a * a + bb * bb) + (c * c + e * e);
     }
   }
-  const float scale = 1.0f / sqrtf(block_sum_ln(q, red) / float(d) + eps);
-  const float *addrow = add ? add + int64_t(sel[seq[r]]) * d : nullptr;
-  // a thread's four consecutive values: 16-byte loads of w, b and the add row, one 16-byte f32 or
-  // 8-byte store per f16 plane
+  const float scale = 1.0f / sqrtf(block_sum_ln(q, red + 4) / float(d) + eps);
+  // a thread's four consecutive values: one 16-byte f32 or 8-byte store per f16 plane
   typedef _Float16 half4_ __attribute__((ext_vector_type(4)));
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < NI; ++i) {
     const int k = threadIdx.x + i * kT;
     if (k >= n4) continue;
     const float in[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-    const float4 w4 = w ? reinterpret_cast<const float4 *>(w)[k] : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-    const float4 b4 = b ? reinterpret_cast<const float4 *>(b)[k] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    const float4 a4 = addrow ? reinterpret_cast<const float4 *>(addrow)[k] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    const float wv[4] = {w4.x, w4.y, w4.z, w4.w}, bv[4] = {b4.x, b4.y, b4.z, b4.w}, av[4] = {a4.x, a4.y, a4.z, a4.w};
+    const float wv[4] = {wr[i].x, wr[i].y, wr[i].z, wr[i].w}, bv[4] = {br[i].x, br[i].y, br[i].z, br[i].w},
+                av[4] = {ar[i].x, ar[i].y, ar[i].z, ar[i].w};
     float4v o;
     half4_ h4, l4;
 #pragma unroll
@@ -413,8 +416,8 @@ void launch_layer_norm(const float *x, const int32_t *rows, int nrows, int d, co
   LG_REQUIRE(nrows > 0 && d > 0 && d % 4 == 0 && d <= 4 * 4 * kT, "layer norm: d=%d outside 4..4096 (multiple of 4)", d);
   LG_REQUIRE((y32 != nullptr) != (y16 != nullptr), "layer norm: exactly one output form");
   LG_REQUIRE(!add || (seq && sel), "layer norm: an add row needs its selectors");
-  hipLaunchKernelGGL(layer_norm_kernel, dim3(nrows), dim3(kT), 0, st, x, rows, d, w, b, eps, add, seq, sel, y16, y16lo,
-                     y32);
+  const auto fn = d <= 4 * kT ? layer_norm_kernel<1> : d <= 8 * kT ? layer_norm_kernel<2> : layer_norm_kernel<4>;
+  hipLaunchKernelGGL(fn, dim3(nrows), dim3(kT), 0, st, x, rows, d, w, b, eps, add, seq, sel, y16, y16lo, y32);
   HIP_CHECK(hipGetLastError());
 }
 
