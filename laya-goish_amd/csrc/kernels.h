@@ -156,16 +156,16 @@ inline float attn_q_scale(int hd) { return 1.4426950408889634f / std::sqrt(float
 
 // Outputs of the q|k|v projection's fused epilogue (launch_gemm_wide_rope): the f32 result
 // (+ bias) is rotated and stored exactly as launch_rope_kv_tiles stores it from the f32 rows.
-// head_dim 128; the launch's output columns are heads col0 / 128 .. of the q|k|v layout (q heads,
-// then k heads, then v heads).
+// The launch's output columns are heads col0 / hd .. of the q|k|v layout (q heads, then k heads, then v
+// heads); head_dim 128, or 64 on the tiles of gemm_mid.h.
 struct RopeKvOut {
-  const float *cosT = nullptr, *sinT = nullptr;          // [ctx][128]
+  const float *cosT = nullptr, *sinT = nullptr;          // [ctx][hd]
   const int32_t *tok_pos = nullptr, *tok_page = nullptr;  // per activation row: position, its page
-  _Float16 *q16 = nullptr, *q16lo = nullptr;              // [M][hq * 128] hi / lo planes
+  _Float16 *q16 = nullptr, *q16lo = nullptr;              // [M][hq * hd] hi / lo planes
   _Float16 *kpool = nullptr, *vpool = nullptr;            // the layer's pools
   int64_t page_stride = 0;                                // as KvGeom::page_stride
-  int hq = 0, hkv = 0, hd = 128, page_tokens = 64, col0 = 0;  // hd: must be 128
-  float qscale = 1.0f;                                    // attn_q_scale(128)
+  int hq = 0, hkv = 0, hd = 128, page_tokens = 64, col0 = 0;
+  float qscale = 1.0f;                                    // attn_q_scale(hd)
   int kv_planes = 2;                                      // 2: hi/lo pool planes; 1: f16 pools
 };
 
