@@ -122,8 +122,8 @@ __global__ __launch_bounds__(kT) void laya_rope_kernel(float *__restrict__ qkv, 
 }
 
 // Bidirectional attention over q|k|v rows [T][3d] (f32, q and k already rotated), head dim 64, on
-// v_mfma_f32_16x16x32_f16 with every f32 operand split into f16 hi + lo parts and three products per pair (hi.hi,
-// lo.hi, hi.lo; lo.lo is below f32 rounding), f32 accumulation.  Keys j with |i - j| <= window (window < 0: the whole
+// v_mfma_f32_16x16x32_f16 with every f32 operand split into f16 hi + lo parts and three products per pair (lo.hi,
+// hi.lo, hi.hi; lo.lo is below f32 rounding), f32 accumulation.  Keys j with |i - j| <= window (window < 0: the whole
 // sequence); scores q.k / sqrt(64) in base 2; online softmax in f32.  Output f16 planes [T][d].
 //
 // One workgroup per (group of at most four consecutive 32-row tiles of one sequence, head): its four waves walk the same
@@ -241,21 +241,29 @@ __global__ __launch_bounds__(256, 2) void laya_attn_kernel(const float *__restri
     for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
       for (int i = 0; i < 4; ++i) s[qb][i / 2][i % 2] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    // the small products of both halves of the head dim first, then the two hi.hi: two roundings at a score's magnitude
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+    for (int ck = 0; ck < 2; ++ck) {
+      f16x8 kh[2][2], kl[2][2];  // [hh][c]
 #pragma unroll
-      for (int ck = 0; ck < 2; ++ck)
+      for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
+        for (int c = 0; c < 2; ++c) {
           const int slot = (ck * 32 + kr0 + 4 * hh) * 8 + ((4 * c + qg) ^ ksw);
-          const f16x8 kh = Kh[slot], kl = Kl[slot];
-#pragma unroll
-          for (int qb = 0; qb < QB; ++qb) {
-            s[qb][ck][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[qb][c], s[qb][ck][hh], 0, 0, 0);
-            s[qb][ck][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[qb][c], s[qb][ck][hh], 0, 0, 0);
-            s[qb][ck][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[qb][c], s[qb][ck][hh], 0, 0, 0);
-          }
+          kh[hh][c] = Kh[slot];
+          kl[hh][c] = Kl[slot];
         }
+#pragma unroll
+      for (int n = 0; n < 6; ++n) {
+        const int c = n % 2;
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+          for (int qb = 0; qb < QB; ++qb)
+            s[qb][ck][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(n < 2 ? kl[hh][c] : kh[hh][c],
+                                                                   n / 2 == 1 ? ql[qb][c] : qh[qb][c], s[qb][ck][hh], 0, 0, 0);
+      }
+    }
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
@@ -288,8 +296,10 @@ __global__ __launch_bounds__(256, 2) void laya_attn_kernel(const float *__restri
         for (int e = 0; e < 4; ++e) mt = fmaxf(mt, s[qb][i / 2][i % 2][e]);
       mt = fmaxf(mt, __shfl_xor(mt, 16));
       mt = fmaxf(mt, __shfl_xor(mt, 32));
-      // the exponent base moves only when a score exceeds it by more than 8; lanes that keep theirs multiply by exactly 1
-      const bool grow = mt > m[qb] + 8.0f;
+      // The exponent base m moves when a score exceeds it by more than 2 (an exponent's rounding grows with its size); lanes
+      // that keep theirs multiply by exactly 1.  Probabilities are held 2^12 times larger (an exact factor that cancels in
+      // O / l), which keeps the lo part of a small one clear of the f16 subnormals' 2^-24 floor; their sum is taken pairwise.
+      const bool grow = mt > m[qb] + 2.0f;
       if (__any(grow)) {
         const float mn = grow ? mt : m[qb];
         const float alpha = __builtin_amdgcn_exp2f(m[qb] - mn);
@@ -300,15 +310,15 @@ __global__ __launch_bounds__(256, 2) void laya_attn_kernel(const float *__restri
           for (int r = 0; r < 4; ++r) acc[qb][b][r] *= alpha;
         m[qb] = mn;
       }
-      float rs = 0.0f;
+      float part[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i) {
+        float4v &p = s[qb][i / 2][i % 2];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float p = __builtin_amdgcn_exp2f(s[qb][i / 2][i % 2][e] - m[qb]);
-          s[qb][i / 2][i % 2][e] = p;
-          rs += p;
-        }
+        for (int e = 0; e < 4; ++e) p[e] = __builtin_amdgcn_exp2f(p[e] - m[qb]) * 4096.0f;
+        part[i] = (p[0] + p[1]) + (p[2] + p[3]);
+      }
+      float rs = (part[0] + part[1]) + (part[2] + part[3]);
       rs += __shfl_xor(rs, 16);
       rs += __shfl_xor(rs, 32);
       lsum[qb] += rs;
@@ -332,9 +342,9 @@ __global__ __launch_bounds__(256, 2) void laya_attn_kernel(const float *__restri
         const f16x8 vh = Vh[slot], vl = Vl[slot];
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
-          acc[qb][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[qb], acc[qb][b], 0, 0, 0);
           acc[qb][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[qb], acc[qb][b], 0, 0, 0);
           acc[qb][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[qb], acc[qb][b], 0, 0, 0);
+          acc[qb][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[qb], acc[qb][b], 0, 0, 0);
         }
       }
     }
