@@ -83,10 +83,11 @@ __global__ __launch_bounds__(kT) void rmsnorm_f16_vec_kernel(const float *__rest
       ss += v[i].z * v[i].z;
       ss += v[i].w * v[i].w;
     }
-  ss = wave_sum_dpp(ss);
+  // block_sum's order: an f16 KV cache turns a last-bit change of the norm into whole f16 steps
+  ss = wave_sum_butterfly(ss);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
-  const float inv = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / float(d) + eps);
+  const float inv = 1.0f / sqrtf((((red[0] + red[1]) + red[2]) + red[3]) / float(d) + eps);
   half4 *out = reinterpret_cast<half4 *>(y + int64_t(blockIdx.x) * d);
   half4 *lo = ylo ? reinterpret_cast<half4 *>(ylo + int64_t(blockIdx.x) * d) : nullptr;
 #pragma unroll

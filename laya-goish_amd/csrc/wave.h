@@ -23,6 +23,22 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
   return ((lane_value(v, 0) + lane_value(v, 16)) + lane_value(v, 32)) + lane_value(v, 48);
 }
 
+// The sum of a shuffle butterfly (lane distances 32, 16, 8, 4, 2, 1), bit for bit, in lane moves: the two long distances
+// swap halves and rows, a rotation of the row by 8 or 4 meets the lane at that distance (after the sum at 8 a row repeats
+// every 8 lanes).  Every lane receives the total.
+__device__ __forceinline__ float wave_sum_butterfly(float v) {
+  typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+  uint2v p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(p.x) + __uint_as_float(p.y);
+  p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(p.x) + __uint_as_float(p.y);
+  v += dpp_move<0x128>(v);  // row_ror:8
+  v += dpp_move<0x124>(v);  // row_ror:4
+  v += dpp_move<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += dpp_move<0xB1>(v);   // quad_perm [1,0,3,2]
+  return v;
+}
+
 }  // namespace lg
 
 namespace lg {

@@ -245,3 +245,39 @@ def test_exact_gemm_deep_k_tilings_agree(lh):
             print(f"openthai-0.8b {name} ({rows} x {cols}) M={M}", flush=True)
             assert_bits_equal(eng.matmul(name, x[:M]), big[:M])
     eng.close()
+
+
+@pytest.mark.parametrize("d", [512, 2048, 3584])
+def test_norm_sum_order(lh, d):
+    """The RMSNorm's sum of squares keeps its order bit for bit (threads over every 1,024th group of four, lanes by halves,
+    then the waves left to right): the f16 KV cache rounds what follows, so another order shows as whole f16 steps.
+    An identity value projection leaves the normalised rows in the cache; embeddings of eight significant bits make
+    every square exact in f32, so that only the order of the sums rounds."""
+    from decoder_image import image
+    rng, n, w = np.random.default_rng(d), 384, 128
+    emb = rng.integers(1, 256, (n, d)) * 2.0 ** rng.integers(-12, -5, (n, d)) * rng.choice([-1.0, 1.0], (n, d))
+    qkv = np.zeros((3 * w, d), np.float32)
+    qkv[2 * w + np.arange(w), np.arange(w)] = 1.0  # v = the first 128 values
+    eng = lh.Engine(lh.Gguf.from_bytes(image(d, 1, 1, w, 128, n, 512, replace={"tok_emb.weight": emb, "qkv.0.weight": qkv})),
+                    kv_tokens=1024)
+    s = eng.seq_create()
+    print(f"norm order d={d}", flush=True)
+    eng.forward(s, np.arange(n), [0], vocab_ids=[0])
+    _, got = eng.seq_kv_read(s, 0, 0, n)
+    eng.close()
+    x = emb.astype(np.float32)
+    part = np.zeros((n, 256), np.float32)
+    for k in range(0, d, 1024):
+        for e in range(4):
+            q = x[:, k + e:min(k + 1024, d):4]
+            part[:, :q.shape[1]] += q * q
+    v = part.reshape(n, 4, 64)
+    for off in (32, 16, 8, 4, 2, 1):
+        v = v + v[:, :, np.arange(64) ^ off]
+    r = v[:, :, 0]
+    ss = ((r[:, 0] + r[:, 1]) + r[:, 2]) + r[:, 3]
+    inv = np.float32(1.0) / np.sqrt(ss / np.float32(d) + np.float32(1e-5))
+    h = x[:, :w] * inv[:, None]
+    hi = h.astype(np.float16)
+    lo = (h - hi.astype(np.float32)).astype(np.float16)
+    assert_bits_equal(got, hi.astype(np.float32) + lo.astype(np.float32))
