@@ -915,12 +915,14 @@ void Engine::run_layers_prefill(BatchPlan &b, lg_cancel_fn cancel, void *arg) {
   ws_h16_.ensure(size_t(T) * d * 2 * planes);
   // q|k|v projections whose GEMM also rotates and stores q, k and v (the exact GEMMs' fused epilogues) leave no f32
   // q|k|v rows to stage
-  auto wide = [&](const ProjPart &p) { return hd == 128 && gemm_wide_takes(T, p.w, Epi::F32); };
-  bool fused = split();
-  for (int l = 0; l < L && fused; ++l)
-    for (const ProjPart &p : layers_[l].qkv)
-      fused = fused && p.col0 % hd == 0 && (wide(p) || gemm_mid_rope_takes(T, p.w, hd));
-  if (!fused) ws_qkv_.ensure(size_t(T) * qkvw * 4);
+  std::vector<uint8_t> fused(L, 0);
+  for (int l = 0; l < L && split(); ++l) {
+    bool rot = true;
+    for (const ProjPart &p : layers_[l].qkv) rot = rot && p.col0 % hd == 0 && std::isfinite(gemm_rope_choice(T, p.w, hd).us);
+    fused[l] = rot;
+  }
+  const bool staged = std::find(fused.begin(), fused.end(), 0) != fused.end();
+  if (staged) ws_qkv_.ensure(size_t(T) * qkvw * 4);
   ws_q16_.ensure(size_t(T) * qw * 2 * planes);
   ws_att16_.ensure(size_t(T) * qw * 2 * planes);
   ws_act16_.ensure(size_t(T) * f * 2 * planes);
@@ -930,7 +932,7 @@ void Engine::run_layers_prefill(BatchPlan &b, lg_cancel_fn cancel, void *arg) {
   _Float16 *q16 = ws_q16_.as<_Float16>(), *q16lo = lo(ws_q16_, int64_t(T) * qw);
   _Float16 *att = ws_att16_.as<_Float16>(), *attlo = lo(ws_att16_, int64_t(T) * qw);
   _Float16 *act = ws_act16_.as<_Float16>(), *actlo = lo(ws_act16_, int64_t(T) * f);
-  float *qkv = fused ? nullptr : ws_qkv_.as<float>();
+  float *qkv = staged ? ws_qkv_.as<float>() : nullptr;
   const KvGeom g = geom();
   prof.begin("embed", stream);
   launch_embed(emb_, emb_kind, b.ids, T, d, V, x, stream);
@@ -957,12 +959,12 @@ void Engine::run_layers_prefill(BatchPlan &b, lg_cancel_fn cancel, void *arg) {
     ro.page_tokens = g.page_tokens;
     ro.qscale = attn_q_scale(hd);
     ro.kv_planes = kv_split() ? 2 : 1;
-    if (fused) {
+    if (fused[l]) {
       for (const ProjPart &p : ly.qkv) {
         ro.col0 = p.col0;
         const _Float16 *ks = chunk_sums(h16, h16lo, T, p.w);
         prof.begin_kernel("gemm");
-        if (!wide(p)) launch_gemm_mid_rope(h16, h16lo, T, p.w, p.bias, ro, stream, ks);
+        if (!gemm_rope_choice(T, p.w, hd).wide) launch_gemm_mid_rope(h16, h16lo, T, p.w, p.bias, ro, stream, ks);
         else if (!launch_gemm_wide_rope(h16, h16lo, T, p.w, p.bias, ro, stream, ks))
           fail(LG_ERR_UNSUPPORTED, "gemm: fused q|k|v launch refused");
         prof.end_kernel(double(p.w.bytes()) + double(T) * p.w.cols * 2, 2.0 * T * double(p.w.rows) * p.w.cols);

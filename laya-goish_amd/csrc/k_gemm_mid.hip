@@ -1,6 +1,7 @@
 // Launches of the exact GEMM tiles of gemm_mid.h, and the choice between them and the 256 x 256 tiles.  Built with
 // MFMA results in VGPRs (-mllvm -amdgpu-mfma-vgpr-form), as k_gemm_q8.hip.
 #include <algorithm>
+#include <cmath>
 
 #include "gemm_mid.h"
 
@@ -32,24 +33,29 @@ constexpr int kHM[kTiles] = {1, 1, 2, 2, 2, 4}, kHN[kTiles] = {1, 2, 2, 4, 4, 4}
 // of K 1024, the others from full rounds)
 constexpr float kWideStep[4] = {3.5f, 2.75f, 4.7f, 3.5f};
 
-// Microseconds of `nk` steps over rounds of two workgroups per CU (the last round alone when half of it or less is left), or
-// of one.
-float cost(const StepCost &c, int64_t tiles, int nk) {
-  const int64_t n = device_cus();
-  if (c.two == 0) return float((tiles + n - 1) / n) * (c.one * nk + c.fill);
+// What the rotating epilogue adds to a round (table reads, eight stores a value pair): measured against the table's
+// costs over F16, Q8_0 and Q4_K q|k|v at 1,100-32,768 rows.
+constexpr float kRopeFill = 2.2f;
+
+// Microseconds of `nk` steps on n CUs over rounds of two workgroups per CU (the last round alone when half of it or less is
+// left), or of one; `extra` a round.
+float cost(const StepCost &c, int64_t n, int64_t tiles, int nk, float extra) {
+  const float fill = c.fill + extra;
+  if (c.two == 0) return float((tiles + n - 1) / n) * (c.one * nk + fill);
   const int64_t rounds = tiles / (2 * n), rest = tiles - rounds * 2 * n;
-  return float(rounds) * (c.two * nk + c.fill) + (rest == 0 ? 0.0f : (rest <= n ? c.one : c.two) * nk + c.fill);
+  return float(rounds) * (c.two * nk + fill) + (rest == 0 ? 0.0f : (rest <= n ? c.one : c.two) * nk + fill);
 }
 
 // The cheapest configuration for M rows of a matrix of `rows` weight rows (only those of 64 columns when rope), and
 // its cost; kNoTile when none divides the output.
 int best_tile(int mode, int M, const DevMatrix &W, bool glu, bool rope, float *best) {
   const int rows = W.rows;
+  const int64_t n = device_cus();
   int t = kNoTile;
   for (int i = 0; i < kTiles; ++i) {
     const int bm = 32 * kHM[i], bn = 32 * kHN[i];
     if (kCost[mode][i].one == 0 || rows % bn || (glu && kHN[i] % 2) || (rope && kHN[i] != 2)) continue;
-    const float c = cost(kCost[mode][i], int64_t((M + bm - 1) / bm) * (rows / bn), W.cols / mid::BK);
+    const float c = cost(kCost[mode][i], n, int64_t((M + bm - 1) / bm) * (rows / bn), W.cols / mid::BK, rope ? kRopeFill : 0.0f);
     if (t == kNoTile || c < *best) {
       t = i;
       *best = c;
@@ -158,23 +164,61 @@ void launch_mode(int mode, int tile, const Launch &l) {
 
 }  // namespace
 
-bool gemm_mid_ahead(int M, const DevMatrix &W, bool glu, int64_t wide_tiles) {
+namespace {
+
+// Whether launch_gemm_mid has the epilogue for weights of `mode`.
+bool mid_epi(int mode, Epi epi) {
+  return epi != Epi::F16 && ((epi != Epi::GEGLU && epi != Epi::RELU16) || mode == W1);
+}
+
+// Microseconds of the tile that a launch takes; infinity when there is none.
+float mid_cost(int M, const DevMatrix &W, bool glu, bool rope) {
   const int mode = mid_mode(M, W);
   float c = 0.0f;
-  if (mode < 0 || best_tile(mode, M, W, glu, false, &c) == kNoTile) return false;
-  // the costs are those of short launches; over more than two rounds of 256 x 256 tiles the card holds its power and the
-  // larger tiles, with fewer instructions an MFMA, win whatever their last round (the 16-request Q4_K/Q6_K
-  // batch, 3.5 rounds of Q6_K down: 31.4 against 34.0 ms), and below that they are given a seventh
-  const int64_t rounds = (wide_tiles + device_cus() - 1) / device_cus();
-  return rounds <= 2 && c * 1.15f < float(rounds) * (kWideStep[mode] * (W.cols / mid::BK) + 1.0f);
+  const int t = best_tile(mode, M, W, glu, rope, &c);
+  return t == kNoTile ? INFINITY : c;
+}
+
+// The 256 x 256 tiles (when takes) or a launch of gemm_mid.h that costs mid_us (infinity: none).  Fewer 256 x 256 tiles than
+// 5/8 of the CUs leaves too many idle.  Between that and one tile per CU they still win (F16 at 1437 rows x 7168 gated,
+// 168 tiles: 47.8 us against 53.4 of the best smaller tiles), and below it they lose.  A last round that is nearly empty
+// loses too (301 rows x 37888 gated F16, 296 tiles, against 170 us), so the modelled costs decide; those are of short
+// launches.  Over more than two rounds the card holds its power and the larger tiles, with fewer instructions an MFMA, win
+// whatever their last round (the 16-request Q4_K/Q6_K batch, 3.5 rounds of Q6_K down: 31.4 against 34.0 ms), and below
+// that they are given a seventh.
+GemmChoice choose(int M, const DevMatrix &W, bool takes, float mid_us) {
+  GemmChoice c{false, mid_us};
+  const int64_t n = device_cus(), tiles = int64_t((M + wide::BM - 1) / wide::BM) * (W.rows / wide::BN);
+  if (!takes || tiles * 8 < n * 5) return c;
+  const int64_t rounds = (tiles + n - 1) / n;
+  const float wide_us = float(rounds) * (kWideStep[wide::prefill_mode(W)] * (W.cols / mid::BK) + 1.0f);
+  if (rounds <= 2 && mid_us * 1.15f < wide_us) return c;
+  return {true, wide_us};
+}
+
+}  // namespace
+
+GemmChoice gemm_choice(int M, const DevMatrix &W, Epi epi) {
+  const int mode = mid_mode(M, W);
+  const bool mid = mode >= 0;
+  return choose(M, W, gemm_wide_takes(M, W, epi), mid ? mid_cost(M, W, epi == Epi::SWIGLU || epi == Epi::GEGLU, false) : INFINITY);
+}
+
+GemmChoice gemm_rope_choice(int M, const DevMatrix &W, int hd) {
+  return choose(M, W, gemm_wide_rope_takes(M, W, hd), gemm_mid_rope_takes(M, W, hd) ? mid_cost(M, W, false, true) : INFINITY);
+}
+
+GemmChoice gemm_laya_rope_choice(int M, const DevMatrix &W, int heads) {
+  return choose(M, W, heads % 2 == 0 && gemm_wide_takes(M, W, Epi::F32),
+                gemm_mid_laya_rope_takes(M, W) ? mid_cost(M, W, false, true) : INFINITY);
 }
 
 bool launch_gemm_mid(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi, float *C,
                      _Float16 *C16, _Float16 *C16lo, int ldc, const float *bias, hipStream_t st, const _Float16 *ks) {
   const int mode = mid_mode(M, W);
   if (mode < 0 || !A || !Alo) return false;
-  const bool glu = epi == Epi::SWIGLU || epi == Epi::GEGLU, f16_only = epi == Epi::GEGLU || epi == Epi::RELU16;
-  if (epi == Epi::F16 || (f16_only && mode != W1)) return false;
+  const bool glu = epi == Epi::SWIGLU || epi == Epi::GEGLU;
+  if (!mid_epi(mode, epi)) return false;
   LG_REQUIRE(mode != WQ4 || ks, "gemm: an exact Q4_K launch needs its activation's chunk sums");
   float c = 0.0f;
   const int tile = best_tile(mode, M, W, glu, false, &c);

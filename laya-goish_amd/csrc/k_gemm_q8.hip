@@ -65,8 +65,8 @@ int device_cus() {
 }
 
 namespace {
-// the wide kernel's mode for W, or -1 when it does not take an M-row launch of W with epilogue
-// EPI (an Epi value or wide::kEpiRopeKv)
+// the wide kernel's mode for W, or -1 when its shape or the epilogue EPI (an Epi value, wide::kEpiRopeKv or
+// wide::kEpiLayaRope) is not one of the wide kernel's
 int wide_mode(int M, const DevMatrix &W, int EPI) {
   using namespace wide;
   const int mode = prefill_mode(W);
@@ -74,17 +74,9 @@ int wide_mode(int M, const DevMatrix &W, int EPI) {
   if (EPI != int(Epi::F32) && EPI != int(Epi::ADD) && EPI != int(Epi::SWIGLU) && EPI != int(Epi::GEGLU) &&
       EPI != kEpiRopeKv && EPI != kEpiLayaRope)
     return -1;
-  const bool glu = EPI == int(Epi::SWIGLU) || EPI == int(Epi::GEGLU);
   const int N = W.rows, K = W.cols;
   if (K % BK != 0 || N % BN != 0) return -1;  // gated: 128 gate + 128 up rows a tile
-  const int NT = glu ? (N / 2) / (BN / 2) : N / BN;
   if (int64_t(N) * K * 2 >= (int64_t(1) << 32)) return -1;  // 32-bit buffer offsets of the weights
-  // fewer 256 x 256 tiles than 5/8 of the CUs leaves too many idle: the smaller tiles fill the device better.  Between
-  // that and one tile per CU the 256 x 256 tiles still win (F16 at 1437 rows x 7168 gated, 168 tiles: 47.8 us against
-  // 53.4 of gemm_mid.h's best), and below it they lose.  A last round that is nearly empty loses too (301 rows x 37888
-  // gated F16, 296 tiles, against 170 us): gemm_mid_ahead compares the rounds.
-  const int64_t tiles = int64_t((M + BM - 1) / BM) * NT;
-  if (tiles * 8 < int64_t(device_cus()) * 5 || gemm_mid_ahead(M, W, glu, tiles)) return -1;
   return mode;
 }
 
@@ -152,12 +144,13 @@ void launch_wide(WideFn fn, int mode, const _Float16 *A, const _Float16 *Alo, in
 
 bool gemm_wide_takes(int M, const DevMatrix &W, Epi epi) { return wide_mode(M, W, int(epi)) >= 0; }
 
+bool gemm_wide_rope_takes(int M, const DevMatrix &W, int hd) { return hd == 128 && wide_mode(M, W, wide::kEpiRopeKv) >= 0; }
+
 bool launch_gemm_wide(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi, float *C,
                       _Float16 *C16, _Float16 *C16lo, int ldc, const float *bias, hipStream_t st, const _Float16 *ks) {
   using namespace wide;
-  if (!A || !Alo) return false;
+  if (!A || !Alo || !gemm_choice(M, W, epi).wide) return false;
   const int mode = wide_mode(M, W, int(epi));
-  if (mode < 0) return false;
   LG_REQUIRE(mode != WQ4 || ks, "gemm: an exact Q4_K launch needs its activation's chunk sums");
   const bool glu = epi == Epi::SWIGLU || epi == Epi::GEGLU;
   const int N = W.rows;
@@ -192,7 +185,7 @@ void launch_gemm_wide_laya_rope(const _Float16 *A, const _Float16 *Alo, int M, c
   using namespace wide;
   LG_REQUIRE(A && Alo && C && cosT && sinT && tok_pos, "gemm laya rope: missing operand");
   const int mode = wide_mode(M, W, kEpiLayaRope);
-  LG_REQUIRE(mode >= 0, "gemm laya rope: the 256 x 256 GEMM does not take %d rows of this matrix", M);
+  LG_REQUIRE(mode >= 0, "gemm laya rope: the 256 x 256 GEMM does not take this matrix");
   LG_REQUIRE(mode != WQ4 || ks, "gemm: an exact Q4_K launch needs its activation's chunk sums");
   LG_REQUIRE(heads > 0 && heads % 2 == 0 && W.rows == 3 * heads * 64 && ldc >= W.rows,
              "gemm laya rope: %d rows are not q|k|v of an even number of 64-dim heads (%d)", W.rows, heads);

@@ -173,13 +173,14 @@ struct RopeKvOut {
 // RoPE and KV cache stores of launch_rope_kv_tiles as its epilogue: q to f16 hi/lo planes
 // (scaled), k and v into the pools (hi/lo planes, or f16 when ro.kv_planes is 1) at each row's
 // position and page.  Returns false (nothing
-// launched) when the wide kernel does not take the launch (gemm_wide_takes) or the layout is not
+// launched) when the wide kernel does not take the launch (gemm_wide_rope_takes) or the layout is not
 // one the epilogue covers (head_dim 128, col0 a multiple of 128).
 bool launch_gemm_wide_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, const float *bias,
                            const RopeKvOut &ro, hipStream_t st, const _Float16 *ks = nullptr);
-// Whether the 256 x 256 exact GEMM takes an M-row launch of W with epilogue epi (shape, prefill
-// copy and tile count; pointers are checked at launch).
+// Whether the 256 x 256 exact GEMM can run an M-row launch of W with epilogue epi, or with the rotating one (shape and
+// prefill copy; pointers are checked at launch).  Whether it is the faster form is gemm_choice's answer.
 bool gemm_wide_takes(int M, const DevMatrix &W, Epi epi);
+bool gemm_wide_rope_takes(int M, const DevMatrix &W, int hd);
 // The encoder's q|k|v projection (W rows: q, k, v of `heads` 64-dim heads, an even count) on the
 // 256 x 256 exact GEMM, its epilogue storing the f32 rows [M][ldc] with q and k rotated: the same bits
 // as the F32 GEMM followed by launch_laya_rope.  Only for launches gemm_wide_takes(M, W, Epi::F32)
@@ -189,8 +190,15 @@ void launch_gemm_wide_laya_rope(const _Float16 *A, const _Float16 *Alo, int M, c
                                 int ldc, hipStream_t st, const _Float16 *ks = nullptr);
 // Compute units of the current device.
 int device_cus();
-// Whether the smaller tiles of gemm_mid.h are ahead of `wide_tiles` 256 x 256 tiles for M rows of W.
-bool gemm_mid_ahead(int M, const DevMatrix &W, bool glu, int64_t wide_tiles);
+// Form of an exact launch over the prefill copy: the 256 x 256 tiles or those of gemm_mid.h, priced over the tiles that the
+// epilogue can run, and its modelled microseconds (infinity: neither takes it).
+struct GemmChoice {
+  bool wide;
+  float us;
+};
+GemmChoice gemm_choice(int M, const DevMatrix &W, Epi epi);
+GemmChoice gemm_rope_choice(int M, const DevMatrix &W, int hd);        // q|k|v of a decoder, rotating epilogue
+GemmChoice gemm_laya_rope_choice(int M, const DevMatrix &W, int heads);  // q|k|v of an encoder, rotating epilogue
 // The two rotating q|k|v launches above on the tiles of gemm_mid.h, for any M the 256 x 256 GEMM does not take, in the
 // exact split mode: the same bits as the F32 GEMM followed by the RoPE kernel.  head_dim 64 or 128, ro.col0 a
 // multiple of it; anything the takes function refuses fails.  The encoder's needs F16 weights.

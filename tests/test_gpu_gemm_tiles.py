@@ -72,3 +72,30 @@ def test_long_vocabulary_argmax(lh):
         eng.seq_free(s)
     assert runs[0] == runs[1]
     eng.close()
+
+
+@pytest.mark.parametrize("preset, layers, counts", [
+    ("f16-7b", 1, (4 * (528,), 8 * (512,), 8 * (672,))), ("q8-2048", 1, (4 * (410,), 7 * (401, 431))),
+    ("q4km-7b", 1, (10 * (440,) + 3 * (131,),)), ("laya-english", 1, (13 * (479,) + 21 * (45,),))])
+def test_qkv_rule_rows(lh, preset, layers, counts):
+    """Row counts where the rotating q|k|v launch goes from the 64-column tiles to the 256 x 256 ones: a request's bits do
+    not change with the launch that its batch takes."""
+    eng = lh.Engine(lh.Gguf.from_bytes(lh.SynthImage(preset, seed=31, n_layers=layers)), kv_tokens=16384)
+    rng = np.random.default_rng(11)
+
+    def run(requests):
+        if preset.startswith("laya"):
+            return [np.concatenate([np.ravel(x) for x in o]) for o in eng.laya_forward([(r, [0, len(r) - 1], 1) for r in requests])]
+        seqs = [eng.seq_create() for _ in requests]
+        out = eng.batch([(s, r, [len(r) - 1]) for s, r in zip(seqs, requests)]).run(np.arange(16, dtype=np.int32))[0]
+        for s in seqs:
+            eng.seq_free(s)
+        return list(out)
+
+    for lengths in counts:
+        ids = [rng.integers(0, 1000, n).astype(np.int32) for n in lengths]
+        whole = run(ids)
+        for i in (0, len(ids) // 2, len(ids) - 1):
+            print(f"{preset} {sum(lengths)} rows, request {i}", flush=True)
+            assert_bits_equal(run([ids[i]])[0], whole[i])
+    eng.close()
