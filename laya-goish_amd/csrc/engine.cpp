@@ -913,13 +913,23 @@ void Engine::run_layers_prefill(BatchPlan &b, lg_cancel_fn cancel, void *arg) {
   const int planes = split() ? 2 : 1;  // hi (+ lo) f16 planes per activation
   ws_x_.ensure(size_t(T) * d * 4);
   ws_h16_.ensure(size_t(T) * d * 2 * planes);
-  // q|k|v projections whose GEMM also rotates and stores q, k and v (the exact GEMMs' fused epilogues) leave no f32
-  // q|k|v rows to stage
+  // q|k|v: GEMMs that also rotate and store q, k and v (no f32 q|k|v rows), or any GEMM to f32 rows and a RoPE pass over
+  // them (10 us and 8 bytes a value at 4.3 TB/s).  The rows' way wins where the rotating epilogue has only 64-column tiles:
+  // head_dim 64 at thousands of rows (F16 2048 x 3072: 2,500 rows 92 us fused against 85, 8,192 314 / 238, 32,768 1211 / 842),
+  // and head_dim 128 just below the 256 x 256 tiles (F16 4608 x 3584: 1,640 rows 179 / 152).  The pass takes up to 40 us more
+  // where a request's length is no multiple of four (16 KV heads of 128: 1,100 rows 109 us fused, 131-144 by rows), hence
+  // the margin at head_dim 128.
+  const float margin = hd == 64 ? 1.1f : 1.25f;
   std::vector<uint8_t> fused(L, 0);
   for (int l = 0; l < L && split(); ++l) {
-    bool rot = true;
-    for (const ProjPart &p : layers_[l].qkv) rot = rot && p.col0 % hd == 0 && std::isfinite(gemm_rope_choice(T, p.w, hd).us);
-    fused[l] = rot;
+    float rot = 0.0f, rows = 10.0f + float(T) * float(qkvw) * (8.0f / 4.3e6f);
+    bool heads = true;
+    for (const ProjPart &p : layers_[l].qkv) {
+      heads = heads && p.col0 % hd == 0;
+      rot += gemm_rope_choice(T, p.w, hd).us;
+      rows += gemm_choice(T, p.w, Epi::F32).us;
+    }
+    fused[l] = heads && std::isfinite(rot) && !(rows * margin < rot);
   }
   const bool staged = std::find(fused.begin(), fused.end(), 0) != fused.end();
   if (staged) ws_qkv_.ensure(size_t(T) * qkvw * 4);

@@ -99,3 +99,32 @@ def test_qkv_rule_rows(lh, preset, layers, counts):
             print(f"{preset} {sum(lengths)} rows, request {i}", flush=True)
             assert_bits_equal(run([ids[i]])[0], whole[i])
     eng.close()
+
+
+def test_head_dim_64_rows(lh):
+    """A head_dim 64 decoder of width 2048: its requests rotate in the q|k|v GEMM, its large batches take the 256 x 256 GEMM and
+    a RoPE pass (the rotating epilogue of that kernel is head_dim 128's), with the same bits."""
+    from decoder_image import image
+    eng = lh.Engine(lh.Gguf.from_bytes(image(2048, 32, 8, 64, 1024, 512, 1024)), kv_tokens=16384)
+    rng = np.random.default_rng(5)
+    options = np.arange(16, dtype=np.int32)
+
+    def run(requests):
+        eng.profile_reset()
+        seqs = [eng.seq_create() for _ in requests]
+        out = eng.batch([(s, r, [len(r) - 1]) for s, r in zip(seqs, requests)]).run(options)[0]
+        for s in seqs:
+            eng.seq_free(s)
+        return out, eng.profile_read("rope_kv")["launches"]
+
+    eng.profile(True)
+    for lengths in (16 * (512,), 9 * (467, 443)):
+        ids = [rng.integers(0, 512, n).astype(np.int32) for n in lengths]
+        print(f"head_dim 64, {sum(lengths)} rows", flush=True)
+        whole, passes = run(ids)
+        assert passes == 1
+        for i in (0, len(ids) - 1):
+            one, passes = run([ids[i]])
+            assert passes == 0
+            assert_bits_equal(one[0], whole[i])
+    eng.close()
