@@ -200,7 +200,7 @@ GemmChoice choose(int M, const DevMatrix &W, bool takes, float mid_us) {
 
 GemmChoice gemm_choice(int M, const DevMatrix &W, Epi epi) {
   const int mode = mid_mode(M, W);
-  const bool mid = mode >= 0;
+  const bool mid = mode >= 0 && mid_epi(mode, epi);
   return choose(M, W, gemm_wide_takes(M, W, epi), mid ? mid_cost(M, W, epi == Epi::SWIGLU || epi == Epi::GEGLU, false) : INFINITY);
 }
 

@@ -235,3 +235,38 @@ def test_kv16_mode_is_the_exact_mode(lh):
         eng.close()
     for a, b in zip(out[0], out[1]):
         assert np.array_equal(np.asarray(a, np.float32).view(np.uint32), np.asarray(b, np.float32).view(np.uint32))
+
+
+def test_quantized_gate_rows(lh, po):
+    """An encoder with Q8_0 gate|up weights: the smaller request tiles have no GeGLU for them, so the choice between tile sizes must
+    not count on those tiles.  A 7,185-row batch (the 256 x 256 kernel) holds its inputs' single results bit for
+    bit, and the oracle's within the bar."""
+    import gguf_writer as gw
+    src = lh.SynthImage("laya-english", seed=8, n_layers=1)  # keeps the image's memory alive
+    og = po.Gguf(src.array())
+    g = lh.Gguf.from_bytes(src)
+    meta = [(k, gw.STR, g.str(k)) for k in ("general.architecture", "general.name", "laya.model_name", "laya.checkpoint",
+                                             "laya.temperature", "laya.temperature_by_options", "ggmlc.graph_spec")]
+    meta += [(k, gw.U32, int(g.num(k))) for k in ("laya.max_opts", "laya.max_len", "laya.head_max_len", "laya.cls_token_id",
+                                                  "laya.sep_token_id", "laya.mask_token_id")]
+    tensors = []
+    for name in g.names():
+        kind, dims, raw = og.tensor(name)
+        if name == "mlp_wi.0.weight":
+            w = np.frombuffer(raw, np.float16).astype(np.float32).reshape(-1, 32)
+            d = (np.abs(w).max(axis=1) / 127).astype(np.float16)
+            codes = np.rint(w / d.astype(np.float32)[:, None]).astype(np.int8)
+            kind, raw = 8, np.concatenate([d.view(np.uint8).reshape(-1, 2), codes.view(np.uint8)], axis=1).tobytes()
+        tensors.append((name, dims, kind, raw))
+    data = np.frombuffer(gw.build(meta, tensors), np.uint8)
+    eng = lh.Engine(lh.Gguf.from_bytes(data))
+    rng = np.random.default_rng(12)
+    inputs = [(rng.integers(0, 50000, 479), [3, 40], i % 3) for i in range(15)]
+    print("Q8_0 gate|up, 15 x 479", flush=True)
+    batch = eng.laya_forward(inputs)
+    for i in (0, 14):
+        (sl, sa), = eng.laya_forward([inputs[i]])
+        assert np.array_equal(batch[i][0], sl) and np.array_equal(batch[i][1], sa)
+    eng.close()
+    wl, wa = po.Laya(po.Gguf(data), threads=8).forward(*inputs[14])
+    assert np.abs(batch[14][0] - wl).max() <= 2e-3 and np.abs(batch[14][1] - wa).max() <= 2e-3
