@@ -922,14 +922,21 @@ void Engine::run_layers_prefill(BatchPlan &b, lg_cancel_fn cancel, void *arg) {
   const float margin = hd == 64 ? 1.1f : 1.25f;
   std::vector<uint8_t> fused(L, 0);
   for (int l = 0; l < L && split(); ++l) {
-    float rot = 0.0f, rows = 10.0f + float(T) * float(qkvw) * (8.0f / 4.3e6f);
-    bool heads = true;
-    for (const ProjPart &p : layers_[l].qkv) {
-      heads = heads && p.col0 % hd == 0;
-      rot += gemm_rope_choice(T, p.w, hd).us;
-      rows += gemm_choice(T, p.w, Epi::F32).us;
+    const std::vector<ProjPart> &parts = layers_[l].qkv;
+    if (l > 0 && std::equal(parts.begin(), parts.end(), layers_[l - 1].qkv.begin(), layers_[l - 1].qkv.end(),
+                            [](const ProjPart &a, const ProjPart &b) { return a.w.kind == b.w.kind && a.w.rows == b.w.rows; })) {
+      fused[l] = fused[l - 1];
+      continue;
     }
-    fused[l] = heads && std::isfinite(rot) && !(rows * margin < rot);
+    float rot = 0.0f, rows = 10.0f + float(T) * float(qkvw) * (8.0f / 4.3e6f), us;
+    bool takes = true;
+    for (const ProjPart &p : parts) {
+      takes = takes && p.col0 % hd == 0 && gemm_rope_form(T, p.w, hd, &us) != GemmForm::None;
+      if (takes) rot += us;
+      gemm_form(T, p.w, Epi::F32, &us);
+      rows += us;
+    }
+    fused[l] = takes && !(rows * margin < rot);
   }
   const bool staged = std::find(fused.begin(), fused.end(), 0) != fused.end();
   if (staged) ws_qkv_.ensure(size_t(T) * qkvw * 4);
@@ -974,7 +981,7 @@ void Engine::run_layers_prefill(BatchPlan &b, lg_cancel_fn cancel, void *arg) {
         ro.col0 = p.col0;
         const _Float16 *ks = chunk_sums(h16, h16lo, T, p.w);
         prof.begin_kernel("gemm");
-        if (!gemm_rope_choice(T, p.w, hd).wide) launch_gemm_mid_rope(h16, h16lo, T, p.w, p.bias, ro, stream, ks);
+        if (gemm_rope_form(T, p.w, hd) == GemmForm::Mid) launch_gemm_mid_rope(h16, h16lo, T, p.w, p.bias, ro, stream, ks);
         else if (!launch_gemm_wide_rope(h16, h16lo, T, p.w, p.bias, ro, stream, ks))
           fail(LG_ERR_UNSUPPORTED, "gemm: fused q|k|v launch refused");
         prof.end_kernel(double(p.w.bytes()) + double(T) * p.w.cols * 2, 2.0 * T * double(p.w.rows) * p.w.cols);

@@ -238,12 +238,12 @@ void Engine::run_laya(BatchPlan &b, const int32_t *qtype_dev, lg_cancel_fn cance
   auto attention = [&](const LayaLayer &y, bool rope) {
     const float *cosT = y.full ? laya_cos_full_ : laya_cos_slide_, *sinT = y.full ? laya_sin_full_ : laya_sin_slide_;
     // the exact GEMMs rotate q and k in their epilogues (the same bits as the RoPE kernel after them)
-    const GemmChoice form = rope && x16lo && hd == 64 ? gemm_laya_rope_choice(T, y.qkv.w, d / hd) : GemmChoice{false, INFINITY};
-    const bool wide = form.wide, fused = std::isfinite(form.us);
+    const GemmForm form = rope && x16lo && hd == 64 ? gemm_laya_rope_form(T, y.qkv.w, d / hd) : GemmForm::None;
+    const bool fused = form != GemmForm::None;
     if (fused) {
       const _Float16 *ks = chunk_sums(x16, x16lo, T, y.qkv.w);
       prof.begin_kernel("gemm");
-      if (wide)
+      if (form == GemmForm::Wide)
         launch_gemm_wide_laya_rope(x16, x16lo, T, y.qkv.w, y.qkv.b, cosT, sinT, b.tok_pos, d / hd, qkv, 3 * d, stream, ks);
       else
         launch_gemm_mid_laya_rope(x16, x16lo, T, y.qkv.w, y.qkv.b, cosT, sinT, b.tok_pos, d / hd, qkv, 3 * d, stream);

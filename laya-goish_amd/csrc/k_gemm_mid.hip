@@ -28,6 +28,15 @@ constexpr StepCost kCost[4][kTiles] = {
     /* W2  */ {{0.26f, 0.50f, 1}, {0.43f, 0.74f, 1}, {0.44f, 0, 2}, {0, 0, 0}, {0.73f, 0, 2}, {1.29f, 0, 6}},
     /* WQ4 */ {{0.24f, 0.40f, 1}, {0.31f, 0.54f, 1}, {0.46f, 0.78f, 2}, {0, 0, 0}, {0.70f, 0, 2}, {1.14f, 0, 3}},
 };
+// What whole layers of 24-32,768 rows measure as a multiple of the table's cost: a launch of several rounds runs at a lower
+// clock and shares L2, most of all where one workgroup fills a CU (F16 3584 x 18944 at 3,000 rows: 892 us for 605).  The table
+// chooses among these tiles; against the 256 x 256 tiles and the RoPE pass this cost counts.
+constexpr float kLong[4][kTiles] = {
+    /* WQ8 */ {1.1f, 1.1f, 1.1f, 1.1f, 1.1f, 1.1f},
+    /* W1  */ {1.06f, 1.06f, 1.06f, 1.1f, 1.4f, 1.3f},
+    /* W2  */ {1.1f, 1.1f, 1.1f, 1.1f, 1.2f, 1.2f},
+    /* WQ4 */ {1.1f, 1.1f, 1.1f, 1.1f, 1.2f, 1.25f},
+};
 constexpr int kHM[kTiles] = {1, 1, 2, 2, 2, 4}, kHN[kTiles] = {1, 2, 2, 4, 4, 4};
 // a 256 x 256 tile's microseconds per 64-deep step, one workgroup per CU (mode order as above; F16 at 168 and 198 tiles
 // of K 1024, the others from full rounds)
@@ -171,46 +180,49 @@ bool mid_epi(int mode, Epi epi) {
   return epi != Epi::F16 && ((epi != Epi::GEGLU && epi != Epi::RELU16) || mode == W1);
 }
 
-// Microseconds of the tile that a launch takes; infinity when there is none.
-float mid_cost(int M, const DevMatrix &W, bool glu, bool rope) {
+// Microseconds of the tile that a launch takes among many rounds; infinity when there is none.
+float long_cost(int M, const DevMatrix &W, bool glu, bool rope) {
   const int mode = mid_mode(M, W);
   float c = 0.0f;
   const int t = best_tile(mode, M, W, glu, rope, &c);
-  return t == kNoTile ? INFINITY : c;
+  return t == kNoTile ? INFINITY : c * kLong[mode][t];
 }
 
-// The 256 x 256 tiles (when takes) or a launch of gemm_mid.h that costs mid_us (infinity: none).  Fewer 256 x 256 tiles than
-// 5/8 of the CUs leaves too many idle.  Between that and one tile per CU they still win (F16 at 1437 rows x 7168 gated,
-// 168 tiles: 47.8 us against 53.4 of the best smaller tiles), and below it they lose.  A last round that is nearly empty
-// loses too (301 rows x 37888 gated F16, 296 tiles, against 170 us), so the modelled costs decide; those are of short
-// launches.  Over more than two rounds the card holds its power and the larger tiles, with fewer instructions an MFMA, win
-// whatever their last round (the 16-request Q4_K/Q6_K batch, 3.5 rounds of Q6_K down: 31.4 against 34.0 ms), and below
-// that they are given a seventh.
-GemmChoice choose(int M, const DevMatrix &W, bool takes, float mid_us) {
-  GemmChoice c{false, mid_us};
+// The 256 x 256 tiles (where they take the launch) or those of gemm_mid.h (where they do); *us, if asked for: the modelled microseconds.  Fewer 256 x 256 tiles than 5/8 of the CUs leaves too many idle.  Between that and one tile per CU they still win (F16 at 1437 rows x 7168 gated, 168 tiles: 47.8 us against 53.4 of the best smaller tiles), and below it they lose.  A last round that is nearly empty
+// loses too (301 rows x 37888 gated F16, 296 tiles, against 170 us), so up to two rounds the modelled costs decide, with 8%
+// for the larger tiles: over 60 shapes and row counts the choice is the faster one or within 4% of it (F16 3584 x 18944 at
+// 3,000 rows 757 us against 892, at 4,800 rows 1623 against 1529; Q4_K 3584 x 3584 at 4,800 rows 371 against 432).  Over more
+// the card holds its power and the larger tiles, with fewer instructions an MFMA, win whatever their last round (the
+// 16-request Q4_K/Q6_K batch, 3.5 rounds of Q6_K down: 31.4 against 34.0 ms).
+GemmForm choose(int M, const DevMatrix &W, bool wide_takes, bool mid_takes, bool glu, bool rope, float *us) {
   const int64_t n = device_cus(), tiles = int64_t((M + wide::BM - 1) / wide::BM) * (W.rows / wide::BN);
-  if (!takes || tiles * 8 < n * 5) return c;
-  const int64_t rounds = (tiles + n - 1) / n;
-  const float wide_us = float(rounds) * (kWideStep[wide::prefill_mode(W)] * (W.cols / mid::BK) + 1.0f);
-  if (rounds <= 2 && mid_us * 1.15f < wide_us) return c;
-  return {true, wide_us};
+  const auto mid_us = [&] { return mid_takes ? long_cost(M, W, glu, rope) : INFINITY; };
+  if (wide_takes && tiles * 8 >= n * 5) {
+    const int64_t rounds = (tiles + n - 1) / n;
+    const float wide_us = float(rounds) * (kWideStep[wide::prefill_mode(W)] * (W.cols / mid::BK) + 1.0f);
+    if (rounds > 2 || !(mid_us() * 1.08f < wide_us)) {
+      if (us) *us = wide_us;
+      return GemmForm::Wide;
+    }
+  }
+  if (us) *us = mid_us();
+  return mid_takes ? GemmForm::Mid : GemmForm::None;
 }
 
 }  // namespace
 
-GemmChoice gemm_choice(int M, const DevMatrix &W, Epi epi) {
+GemmForm gemm_form(int M, const DevMatrix &W, Epi epi, float *us) {
   const int mode = mid_mode(M, W);
-  const bool mid = mode >= 0 && mid_epi(mode, epi);
-  return choose(M, W, gemm_wide_takes(M, W, epi), mid ? mid_cost(M, W, epi == Epi::SWIGLU || epi == Epi::GEGLU, false) : INFINITY);
+  return choose(M, W, gemm_wide_takes(M, W, epi), mode >= 0 && mid_epi(mode, epi), epi == Epi::SWIGLU || epi == Epi::GEGLU,
+                false, us);
 }
 
-GemmChoice gemm_rope_choice(int M, const DevMatrix &W, int hd) {
-  return choose(M, W, gemm_wide_rope_takes(M, W, hd), gemm_mid_rope_takes(M, W, hd) ? mid_cost(M, W, false, true) : INFINITY);
+GemmForm gemm_rope_form(int M, const DevMatrix &W, int hd, float *us) {
+  return choose(M, W, gemm_wide_rope_takes(M, W, hd), gemm_mid_rope_takes(M, W, hd), false, true, us);
 }
 
-GemmChoice gemm_laya_rope_choice(int M, const DevMatrix &W, int heads) {
-  return choose(M, W, heads % 2 == 0 && gemm_wide_takes(M, W, Epi::F32),
-                gemm_mid_laya_rope_takes(M, W) ? mid_cost(M, W, false, true) : INFINITY);
+GemmForm gemm_laya_rope_form(int M, const DevMatrix &W, int heads) {
+  return choose(M, W, heads % 2 == 0 && gemm_wide_takes(M, W, Epi::F32), gemm_mid_laya_rope_takes(M, W), false, true, nullptr);
 }
 
 bool launch_gemm_mid(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi, float *C,

@@ -149,7 +149,7 @@ bool gemm_wide_rope_takes(int M, const DevMatrix &W, int hd) { return hd == 128 
 bool launch_gemm_wide(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi, float *C,
                       _Float16 *C16, _Float16 *C16lo, int ldc, const float *bias, hipStream_t st, const _Float16 *ks) {
   using namespace wide;
-  if (!A || !Alo || !gemm_choice(M, W, epi).wide) return false;
+  if (!A || !Alo || gemm_form(M, W, epi) != GemmForm::Wide) return false;
   const int mode = wide_mode(M, W, int(epi));
   LG_REQUIRE(mode != WQ4 || ks, "gemm: an exact Q4_K launch needs its activation's chunk sums");
   const bool glu = epi == Epi::SWIGLU || epi == Epi::GEGLU;

@@ -178,7 +178,7 @@ struct RopeKvOut {
 bool launch_gemm_wide_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, const float *bias,
                            const RopeKvOut &ro, hipStream_t st, const _Float16 *ks = nullptr);
 // Whether the 256 x 256 exact GEMM can run an M-row launch of W with epilogue epi, or with the rotating one (shape and
-// prefill copy; pointers are checked at launch).  Whether it is the faster form is gemm_choice's answer.
+// prefill copy; pointers are checked at launch).  Whether it is the faster form is gemm_form's answer.
 bool gemm_wide_takes(int M, const DevMatrix &W, Epi epi);
 bool gemm_wide_rope_takes(int M, const DevMatrix &W, int hd);
 // The encoder's q|k|v projection (W rows: q, k, v of `heads` 64-dim heads, an even count) on the
@@ -191,14 +191,11 @@ void launch_gemm_wide_laya_rope(const _Float16 *A, const _Float16 *Alo, int M, c
 // Compute units of the current device.
 int device_cus();
 // Form of an exact launch over the prefill copy: the 256 x 256 tiles or those of gemm_mid.h, priced over the tiles that the
-// epilogue can run, and its modelled microseconds (infinity: neither takes it).
-struct GemmChoice {
-  bool wide;
-  float us;
-};
-GemmChoice gemm_choice(int M, const DevMatrix &W, Epi epi);
-GemmChoice gemm_rope_choice(int M, const DevMatrix &W, int hd);        // q|k|v of a decoder, rotating epilogue
-GemmChoice gemm_laya_rope_choice(int M, const DevMatrix &W, int heads);  // q|k|v of an encoder, rotating epilogue
+// epilogue can run (None: neither takes it); *us, when asked for, gets its modelled microseconds (infinity for None).
+enum class GemmForm { None, Mid, Wide };
+GemmForm gemm_form(int M, const DevMatrix &W, Epi epi, float *us = nullptr);
+GemmForm gemm_rope_form(int M, const DevMatrix &W, int hd, float *us = nullptr);  // q|k|v of a decoder, rotating epilogue
+GemmForm gemm_laya_rope_form(int M, const DevMatrix &W, int heads);               // q|k|v of an encoder, rotating epilogue
 // The two rotating q|k|v launches above on the tiles of gemm_mid.h, for any M the 256 x 256 GEMM does not take, in the
 // exact split mode: the same bits as the F32 GEMM followed by the RoPE kernel.  head_dim 64 or 128, ro.col0 a
 // multiple of it; anything the takes function refuses fails.  The encoder's needs F16 weights.
