@@ -130,15 +130,19 @@ __global__ __launch_bounds__(kT) void laya_rope_kernel(float *__restrict__ qkv, 
 // 64-key blocks (aligned to the sequence's start, so a query's arithmetic depends on its position only), and each
 // block's K and V rows are read, split and staged in LDS once for up to 128 queries, V transposed, the next block's rows
 // on their way in registers.  (The former form gave every 16 queries a workgroup that read and split all keys
-// again, on the 16x16x16 instruction: 699 us a full and ~380 a windowed layer of 64 inputs of 473-512 tokens, against 210
-// and ~165.)  QB 16-query blocks a wave: 2, a wave takes a tile; 1, half a tile, two workgroups (z) a group, when whole
+// again, on the 16x16x16 instruction: 657 us a full and 301 a windowed layer of 64 inputs of 492 tokens, 12 heads, against
+// 207 and 125.)  QB 16-query blocks a wave: 2, a wave takes a tile; 1, half a tile, two workgroups (z) a group, when whole
 // groups would leave CUs idle.
 // S^T = K Q^T in 16 x 16 blocks: lane l feeds row lr = l % 16 of key block (ck, hh), which is key ck * 32 + 8 (lr / 4) + 4 hh +
 // lr % 4, so that it receives, for query lr, keys ck * 32 + 8 qg + 4 hh + 0..3, qg = l / 16: blocks (ck, 0) and (ck, 1)
 // together are the eight keys its P^T operand of O^T = V^T P^T takes (the decoder's prefill attention has the same form).
+// Rounding: a block's output is summed from zero, its small products first, and added to the running O once, so O is rounded
+// once per 64 keys and not with each of six products (an MFMA's own sum truncates).  The exponent is one fused operation on the
+// raw score.  Error against 64 bits over 492-token inputs, this form / one chain with a rounded product / the former four
+// chains of a quarter of the keys: flat scores 4.0 / 4.6 / 4.1 e-7, scores of deviation 4 3.8 / 4.6 / 5.1 e-7; the same time.
 // LDS: 16-byte chunk x of a K row at slot x ^ kswz(row); V rows (one dim, 64 keys) with one pad slot: operand reads
 // without bank conflicts.
-// scores in base-2 units; applied to them and not to q, whose f16 range stays the operand's own
+// scores to base-2 units; applied to them and not to q, whose f16 range stays the operand's own
 constexpr float kScoreLog2 = 0.125f * 1.44269504088896341f;
 constexpr int kKB = 64;                     // keys per block
 constexpr int kKSlots = kKB * 8, kVSlots = kHD * 9;  // 16-byte slots of a plane
@@ -264,12 +268,6 @@ __global__ __launch_bounds__(256, 2) void laya_attn_kernel(const float *__restri
                                                                    n / 2 == 1 ? ql[qb][c] : qh[qb][c], s[qb][ck][hh], 0, 0, 0);
       }
     }
-#pragma unroll
-    for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s[qb][i / 2][i % 2][e] *= kScoreLog2;
     if (k0 + kKB > n || (window >= 0 && (k0 + kKB - 1 - pos0 > window || pos0 + 16 * QB - 1 - k0 > window))) {
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
@@ -296,6 +294,7 @@ __global__ __launch_bounds__(256, 2) void laya_attn_kernel(const float *__restri
         for (int e = 0; e < 4; ++e) mt = fmaxf(mt, s[qb][i / 2][i % 2][e]);
       mt = fmaxf(mt, __shfl_xor(mt, 16));
       mt = fmaxf(mt, __shfl_xor(mt, 32));
+      mt *= kScoreLog2;
       // The exponent base m moves when a score exceeds it by more than 2 (an exponent's rounding grows with its size); lanes
       // that keep theirs multiply by exactly 1.  Probabilities are held 2^12 times larger (an exact factor that cancels in
       // O / l), which keeps the lo part of a small one clear of the f16 subnormals' 2^-24 floor; their sum is taken pairwise.
@@ -315,7 +314,7 @@ __global__ __launch_bounds__(256, 2) void laya_attn_kernel(const float *__restri
       for (int i = 0; i < 4; ++i) {
         float4v &p = s[qb][i / 2][i % 2];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) p[e] = __builtin_amdgcn_exp2f(p[e] - m[qb]) * 4096.0f;
+        for (int e = 0; e < 4; ++e) p[e] = __builtin_amdgcn_exp2f(fmaf(p[e], kScoreLog2, -m[qb])) * 4096.0f;
         part[i] = (p[0] + p[1]) + (p[2] + p[3]);
       }
       float rs = (part[0] + part[1]) + (part[2] + part[3]);
@@ -323,30 +322,40 @@ __global__ __launch_bounds__(256, 2) void laya_attn_kernel(const float *__restri
       rs += __shfl_xor(rs, 32);
       lsum[qb] += rs;
     }
+    f16x8 ph[QB][2], pl[QB][2];
 #pragma unroll
-    for (int ck = 0; ck < 2; ++ck) {
-      f16x8 ph[QB], pl[QB];
+    for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-      for (int qb = 0; qb < QB; ++qb) {
+      for (int ck = 0; ck < 2; ++ck) {
         float pv[8];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           pv[e] = s[qb][ck][0][e];
           pv[4 + e] = s[qb][ck][1][e];
         }
-        split8_pk(pv, ph[qb], pl[qb]);
+        split8_pk(pv, ph[qb][ck], pl[qb][ck]);
       }
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
+    for (int b = 0; b < 4; ++b) {
+      f16x8 vh[2], vl[2];
+#pragma unroll
+      for (int ck = 0; ck < 2; ++ck) {
         const int slot = (b * 16 + lr) * 9 + 4 * ck + qg;
-        const f16x8 vh = Vh[slot], vl = Vl[slot];
-#pragma unroll
-        for (int qb = 0; qb < QB; ++qb) {
-          acc[qb][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[qb], acc[qb][b], 0, 0, 0);
-          acc[qb][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[qb], acc[qb][b], 0, 0, 0);
-          acc[qb][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[qb], acc[qb][b], 0, 0, 0);
-        }
+        vh[ck] = Vh[slot];
+        vl[ck] = Vl[slot];
       }
+      float4v t[QB];
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) t[qb] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int n = 0; n < 6; ++n)
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb)
+          t[qb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(n < 2 ? vl[n % 2] : vh[n % 2], n / 2 == 1 ? pl[qb][n % 2] : ph[qb][n % 2], t[qb], 0, 0, 0);
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[qb][b][r] += t[qb][r];
     }
   }
   if (!active) return;

@@ -270,3 +270,43 @@ def test_quantized_gate_rows(lh, po):
     eng.close()
     wl, wa = po.Laya(po.Gguf(data), threads=8).forward(*inputs[14])
     assert np.abs(batch[14][0] - wl).max() <= 2e-3 and np.abs(batch[14][1] - wa).max() <= 2e-3
+
+
+def test_attention_sum_error(lh, po):
+    """The attention's running sum: values of +16 in the first half of a sequence and -16 in the second nearly cancel, so that
+    every rounding at the running sum's size shows 150-fold in the output.  A block of 64 keys is summed by itself and added
+    once, so a 512-token sequence has eight such roundings of at most 2^-24 each at no more than half the offset: about 1e-5 of
+    the outputs (one chain through all keys, three products a 32-key step: 3e-5).  Against float64 with the bound at 1.5e-5."""
+    import np_laya
+    src = lh.SynthImage("laya-tiny", seed=13)  # keeps the image's memory alive
+    arr = src.array().copy()
+    og = po.Gguf(arr)
+    d, rng = 128, np.random.default_rng(21)
+
+    def put(name, values):
+        kind, dims, _ = og.tensor(name)
+        assert kind == 1 and list(dims) == list(values.shape[::-1]), name
+        off = og.offset(name)
+        arr[off:off + values.size * 2] = np.ascontiguousarray(values, np.float16).view(np.uint8).ravel()
+
+    emb = rng.standard_normal((1024, d))
+    emb[:, d - 1] = np.where(np.arange(1024) < 512, 1.0, -1.0)
+    qkv = np.concatenate([0.02 * rng.standard_normal((2 * d, d)), np.eye(d)])
+    qkv[2 * d:, d - 1] += 16.0
+    put("tok_emb.weight", emb)
+    put("qkv.0.weight", qkv)
+    put("wo.0.weight", 256.0 * np.eye(d))
+    for name in lh.Gguf.from_bytes(src).names():
+        if name.startswith(("wo.", "mlp_wo.", "head_wo.", "head_fc2.")) and name.endswith(".weight") and name != "wo.0.weight":
+            put(name, np.zeros(og.tensor(name)[1][::-1]))
+    eng = lh.Engine(lh.Gguf.from_bytes(arr))
+    inputs = [(np.concatenate([rng.integers(0, 512, 256), rng.integers(512, 1024, 256)]), sorted(rng.choice(512, 16, replace=False).tolist()), 0)
+              for _ in range(12)]
+    print("attention sums, 12 x 512", flush=True)
+    got = np.stack([l for l, _ in eng.laya_forward(inputs)]).astype(np.float64)
+    eng.close()
+    om = np_laya.F64Laya(og)
+    want = np.stack([om.forward(*x)[0] for x in inputs])
+    err = np.linalg.norm(got - want) / np.linalg.norm(want - want.mean(axis=0))
+    print(f"relative error {err:.2e}", flush=True)
+    assert err <= 1.5e-5
