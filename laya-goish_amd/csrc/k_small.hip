@@ -764,6 +764,7 @@ void launch_head_rows(const float *x, const int32_t *rows, int R, int d, const f
                       float *logits, hipStream_t st) {
   LG_REQUIRE(R > 0 && nv > 0 && W.cols == d, "head: bad shape");
   LG_REQUIRE(d % 8 == 0, "head: d=%d is not a multiple of 8", d);
+  LG_REQUIRE(d <= 16384, "head: d=%d is past the widths that forwards take", d);
   // a few rows: one row and one option a wave, every load of the row in flight; from 16 rows blocks of four by four
   if (R < 16) launch_head_kind<1, 1>(x, rows, R, d, norm_w, eps, W, bias, vocab_ids, nv, logits, st);
   else launch_head_kind<4, 4>(x, rows, R, d, norm_w, eps, W, bias, vocab_ids, nv, logits, st);

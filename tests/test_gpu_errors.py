@@ -83,3 +83,18 @@ def test_non_finite_output_is_an_error(lh, po):
         eng.decode(s, 1, 3)
     assert eng.seq_len(s) == 40
     eng.close()
+
+
+def test_width_limit_of_option_rows(lh):
+    """A decoder wider than 16,384 loads, but its option rows are refused, in a forward and in a batch, as before the head
+    took them in one pass."""
+    from decoder_image import image
+    d = 16512
+    eng = lh.Engine(lh.Gguf.from_bytes(image(d, 2, 1, 64, 64, 128, 128)), kv_tokens=256)
+    ids = np.arange(5, dtype=np.int32)
+    print("width 16512", flush=True)
+    with pytest.raises(lh.LayaError, match="head: d"):
+        eng.forward(eng.seq_create(), ids, [4], [1, 2])
+    with pytest.raises(lh.LayaError, match="head: d"):
+        eng.batch([(eng.seq_create(), ids, [4])]).run([1, 2])
+    eng.close()
