@@ -128,3 +128,66 @@ def test_head_dim_64_rows(lh):
             assert passes == 0
             assert_bits_equal(one[0], whole[i])
     eng.close()
+
+
+@pytest.mark.parametrize("zeroed", [0, 40000])
+def test_long_argmax_ties(lh, zeroed):
+    """Equal maxima in several of the 64 ranges of a long vocabulary: the first one wins (src/models/openthai/decision.rs:330-335).
+    With the rows below 40,000 zeroed, which ends inside a range, it is token 0 or 40,000 by the sign of the others."""
+    from decoder_image import image
+    V, d = 66048, 256
+    head = np.tile(np.random.default_rng(2).standard_normal(d) * 0.05, (V, 1))
+    head[:zeroed] = 0
+    eng = lh.Engine(lh.Gguf.from_bytes(image(d, 2, 1, 128, 256, V, 256, replace={"output.weight": head})), kv_tokens=512)
+    s = eng.seq_create()
+    eng.forward(s, [3, 4, 5], [2], [0])
+    toks, logits = eng.decode(s, 6, 6, want_logits=True)
+    for t, z in zip(toks, logits):
+        assert (z[zeroed:] == z[V - 1]).all() and z[V - 1] != 0
+        assert int(t) == (zeroed if z[V - 1] > 0 else 0) == int(np.argmax(z))
+    eng.close()
+
+
+def test_long_argmax_non_finite(lh):
+    """A long vocabulary whose maximum is infinite has no token: the decode fails and the engine stays usable."""
+    from decoder_image import image
+    V, d = 66048, 256
+    head = np.random.default_rng(3).standard_normal((V, d)) * 0.05
+    head[50000, 0], head[50001, 0] = np.inf, -np.inf  # one of the two is +inf whatever the sign of its input
+    eng = lh.Engine(lh.Gguf.from_bytes(image(d, 2, 1, 128, 256, V, 256, replace={"output.weight": head})), kv_tokens=512)
+    s = eng.seq_create()
+    eng.forward(s, [3, 4, 5], [2], [0])
+    with pytest.raises(lh.LayaError, match="non-finite model output"):
+        eng.decode(s, 6, 3)
+    assert eng.seq_len(s) == 3
+    assert np.isfinite(eng.forward(s, [7, 8], [1], [1, 2])).all()
+    eng.close()
+
+
+@pytest.mark.parametrize("preset, precision", [("plumbing-f16", 0), ("q8-2048", 2), ("q4km-7b", 0)])
+@pytest.mark.parametrize("prefix", [5, 37, 100])
+def test_attention_tiles_behind_a_prefix(lh, preset, precision, prefix):
+    """Requests behind a cached prefix that ends inside a page and inside a tile: alone they take 16-row attention tiles, in a
+    batch 32-row ones, with the same bits."""
+    eng = lh.Engine(lh.Gguf.from_bytes(lh.SynthImage(preset, seed=31, n_layers=1)), kv_tokens=32768,
+                    precision=lh.PREC_KV16 if precision else lh.PREC_EXACT)
+    rng = np.random.default_rng(prefix)
+    base = eng.seq_create()
+    eng.forward(base, rng.integers(0, 1000, prefix).astype(np.int32), [0], vocab_ids=[0])
+    ids = [rng.integers(0, 1000, n).astype(np.int32) for n in (1, 15, 16, 17, 31, 33, 64, 97, 300)]
+    options = np.arange(16, dtype=np.int32)
+
+    def run(requests):
+        seqs = [eng.seq_fork(base, prefix) for _ in requests]
+        out = eng.batch([(s, r, [len(r) // 2, len(r) - 1] if len(r) > 1 else [0]) for s, r in zip(seqs, requests)]).run(options)[0]
+        for s in seqs:
+            eng.seq_free(s)
+        return out
+
+    whole, at = run(ids * 8), 0
+    for r in ids:
+        n = 2 if len(r) > 1 else 1
+        print(f"{preset} {len(r)} tokens behind {prefix}", flush=True)
+        assert_bits_equal(run([r]), whole[at:at + n])
+        at += n
+    eng.close()
