@@ -753,7 +753,7 @@ BatchPlan *Engine::batch_create(const lg_request *reqs, int nreq) {
   try {
     std::vector<int32_t> ids, tseq, tpos, tpage, tiles_s, tiles_r, tiles_p, tiles_n, gather, grp_f, grp_c, srow0, sn;
     std::vector<int32_t> it_r, it_p, it_n, it_lo, it_hi, cb_r, cb_n, cb_f, cb_c;
-    int max_pages = 0, max_len = 0;  // max_len: the longest sequence of the batch once its tokens are in
+    int max_pages = 0;
     for (int r = 0; r < nreq; ++r) {
       const lg_request &q = reqs[r];
       Seq &s = seq(q.seq);
@@ -770,12 +770,14 @@ BatchPlan *Engine::batch_create(const lg_request *reqs, int nreq) {
              r, q.seq, s.len);
       if (s.len + q.n > ctx) fail(LG_ERR_INVALID, "request %d: %d tokens exceed the context length %d", r, s.len + q.n, ctx);
       if (!fresh) max_pages = std::max(max_pages, (s.len + q.n + 63) / 64);
-      max_len = std::max(max_len, s.len + q.n);
     }
     if (arch == Arch::Decoder) {
-      std::vector<int32_t> fresh_n;
-      for (int r = 0; r < nreq; ++r) fresh_n.push_back(reqs[r].n);
-      b->tiling = attn_prefill_tiling(hq, hkv, max_len, fresh_n.data(), nreq);
+      std::vector<int32_t> start, added;
+      for (int r = 0; r < nreq; ++r) {
+        start.push_back(seq(reqs[r].seq).len);
+        added.push_back(reqs[r].n);
+      }
+      b->tiling = attn_prefill_tiling(hq, geom(), start.data(), added.data(), nreq);
     }
     const int gtiles = b->tiling.group_tiles, trows = b->tiling.tile_rows;
     const int64_t T = std::accumulate(reqs, reqs + nreq, int64_t(0), [](int64_t a, const lg_request &q) { return a + q.n; });

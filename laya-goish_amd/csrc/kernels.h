@@ -230,9 +230,8 @@ void launch_rope_kv_tiles(const float *qkv, int hq, const KvGeom &g, const float
 struct AttnTiling {
   int tile_rows = 32, group_tiles = 4;
 };
-// The tiling of a batch whose sequences get new_tokens[i] tokens each (max_len: the longest sequence of the batch, its
-// own tokens included).
-AttnTiling attn_prefill_tiling(int hq, int hkv, int max_len, const int32_t *new_tokens, int nseq);
+// The tiling of a batch whose sequences hold start[i] tokens and get new_tokens[i] more.
+AttnTiling attn_prefill_tiling(int hq, const KvGeom &g, const int32_t *start, const int32_t *new_tokens, int nseq);
 void launch_attn_prefill(const _Float16 *q16, const _Float16 *q16_lo, int T, int hq,
                          const KvGeom &g, const void *kpool, const void *vpool,
                          const int32_t *pages, int max_pages, const int32_t *tile_seq,
