@@ -24,8 +24,8 @@
 // (ping-pong, below), one barrier per half step.
 //
 // LDS rows are 64 bytes (four 16-byte chunks); logical chunk c of row r sits in slot
-// c ^ ((r >> 2) & 3), so the 16 lanes of each quarter of an operand read (16 rows, one chunk)
-// fall in 16 distinct 16-byte bank groups.  The DMA side writes whole 1 KiB blocks: lane L of a
+// c ^ ((r >> 1) & 3), so the eight lanes that one pass of an operand read serves (rows r .. r + 7, one
+// chunk) fall in the eight 16-byte groups of 128 bytes.  The DMA side writes whole 1 KiB blocks: lane L of a
 // block fetches the global chunk that belongs in its slot.
 #pragma once
 #include <hip/hip_runtime.h>

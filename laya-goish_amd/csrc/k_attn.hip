@@ -43,22 +43,21 @@ constexpr int P = 64;  // tokens per page
 #define MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_f16((a), (b), (c), 0, 0, 0)
 
 // Prefill.  Work item: (tile group, kv head kh, head block hb).  A tile group is <= T
-// consecutive 32-query tiles of one sequence, a head block GB consecutive query heads of kh's
+// consecutive tiles of 16 QB queries of one sequence, a head block GB consecutive query heads of kh's
 // group of G = hq / hkv.  Wave w computes head kh * G + hb * GB + w % GB on tile w / GB of the
 // group, so all W = GB * T waves read the same K/V pages: each page passes through LDS once per
-// workgroup.  Pages are copied global -> LDS by LDS-DMA loads (16 bytes a lane, no registers),
-// double-buffered: page kt + 1 is in flight while page kt is consumed, one barrier per page.
+// workgroup.  Pages are copied global -> LDS by LDS-DMA loads (16 bytes a lane, no registers) into STG
+// stages.
 //
 // S^T = K . Q^T on MFMA 16x16x32 f16 (one instruction per 32-deep chunk of the head dim), keys as
-// rows and queries as columns, in 16 x 16 blocks: a wave's 32 queries are two query blocks qb, a
-// page's 64 keys four key blocks (ck, h) of two 32-key chunks ck.  Lane l feeds row r = l % 16 of a
+// rows and queries as columns, in 16 x 16 blocks: a wave's queries are QB query blocks qb, a page's
+// 64 keys four key blocks (ck, h) of two 32-key chunks ck.  Lane l feeds row r = l % 16 of a
 // key block, and row r of block (ck, h) is key ck * 32 + 8 (r / 4) + 4 h + r % 4: the result leaves
 // lane l (query l % 16 of its block) with keys ck * 32 + 8 g + 4 h + 0..3, g = l / 16, so its scores
 // of (ck, 0) and (ck, 1) together are the eight keys ck * 32 + 8 g + 0..7 that its P^T operand of
 // O^T = V^T . P^T takes against one 16-byte run of a V row.  A query's 64 scores of a page sit in the
-// four lanes l % 16 + 16 g; the online softmax reduces over them with two lane swaps.  Each wave
-// runs eight independent score chains and sixteen output chains, so no MFMA waits on the one
-// before it.
+// four lanes l % 16 + 16 g; the online softmax reduces over them with two lane swaps.  Each wave runs
+// 4 QB independent score chains and QB hd / 16 output chains, so an MFMA seldom waits on the one before it.
 // LDS: K rows unpadded, the 16-byte chunk x of key row R at slot x ^ kswz(R), so the sixteen rows
 // an operand read takes fall in distinct 16-byte bank groups; V rows (one dim, 64 keys) carry one
 // pad slot for the same reason.

@@ -8,14 +8,16 @@ namespace {
 template <uint32_t KIND>
 void launch_kind(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi, float *C,
                  _Float16 *C16, _Float16 *C16lo, int ldc, const float *bias, hipStream_t st, const _Float16 *ks) {
-  // Chosen by sweeps at the 35,840-token Q8_0/F16 and 32,768-token Q4_K/Q6_K 7B prefill
+  // FAST mode: chosen by sweeps at the 35,840-token Q8_0/F16 and 32,768-token Q4_K/Q6_K 7B prefill
   // shapes; a 256-wide N tile falls back to 128 when it does not divide the output width.
   if (!Alo) {
     if (launch_cfg<KIND, FAST, 64, 8, 8, 1>(A, Alo, M, W, epi, C, C16, C16lo, ldc, bias, st)) return;
     if (launch_cfg<KIND, FAST, 64, 4, 4, 2>(A, Alo, M, W, epi, C, C16, C16lo, ldc, bias, st)) return;
   } else if (launch_gemm_wide(A, Alo, M, W, epi, C, C16, C16lo, ldc, bias, st, ks) ||
              launch_gemm_mid(A, Alo, M, W, epi, C, C16, C16lo, ldc, bias, st, ks)) {
-    return;  // below: matrices without a prefill copy (the head and the single tensors of lg_matmul)
+    return;
+  // below: matrices without a prefill copy (the single tensors of lg_matmul), an encoder's quantised gate|up and ReLU
+  // weights where the 256 x 256 tiles are too few, and planes of 4 GiB and more
   } else if (KIND == LG_Q4_K && needs_ksum(W)) {
     if (launch_gemm_q4_exact(A, Alo, M, W, epi, C, C16, C16lo, ldc, bias, st, ks)) return;
   } else if constexpr (KIND == LG_Q8_0) {
@@ -27,9 +29,8 @@ void launch_kind(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix 
     const bool glu = epi == Epi::SWIGLU || epi == Epi::GEGLU;
     const int outN = glu ? W.rows / 2 : W.rows;
     const int64_t tiles = int64_t((M + 127) / 128) * (outN / (glu ? 64 : 128));
-    // few 64 x 64 tiles (a short request): 32 x 32 tiles (32 x 64 weight rows for gate|up) over two LDS
-    // stages, four times the workgroups and a quarter of each K step's LDS traffic per workgroup (C1's
-    // 144-token request 0.49-0.51 -> 0.40 ms; 128-deep K steps with one stage 0.41-0.43, 64-deep 0.45)
+    // few 64 x 64 tiles (a few dozen rows): 32 x 32 tiles (32 x 64 weight rows for gate|up) over two LDS
+    // stages, four times the workgroups and a quarter of each K step's LDS traffic per workgroup
     if (int64_t((M + 63) / 64) * (outN / 64) < 128 && W.cols % 128 == 0 &&
         (glu ? launch_cfg<KIND, SPLIT, 128, 1, 2, 2>(A, Alo, M, W, epi, C, C16, C16lo, ldc, bias, st)
              : launch_cfg<KIND, SPLIT, 128, 1, 1, 2>(A, Alo, M, W, epi, C, C16, C16lo, ldc, bias, st)))
@@ -49,9 +50,8 @@ void launch_kind(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix 
     if (tiles < 256 && launch_cfg<KIND, SPLIT, 64, 2, 4, 1>(A, Alo, M, W, epi, C, C16, C16lo, ldc, bias, st)) return;
     if (launch_cfg<KIND, SPLIT, 64, 4, 4, 1>(A, Alo, M, W, epi, C, C16, C16lo, ldc, bias, st)) return;
   } else {
-    // short launches, as the exact Q8_0 and Q4_K tiles (a 144-token request on two layers of the Q4_K/Q6_K
-    // 7B shape 2.43 -> 1.77 ms, 560 tokens 2.75 -> 2.17 ms, 1024 tokens 3.29 -> 3.21 ms).  Q4_K weights
-    // are dequantised in 64-deep steps of 32-element chunks, so their tiles are at least 128 columns wide.
+    // short launches, as the exact Q8_0 and Q4_K tiles.  Q4_K weights are dequantised in 64-deep steps of
+    // 32-element chunks, so their tiles are at least 128 columns wide.
     {
       const bool glu = epi == Epi::SWIGLU || epi == Epi::GEGLU;
       const int outN = glu ? W.rows / 2 : W.rows;

@@ -13,10 +13,9 @@ namespace lg {
 bool launch_gemm_q8_exact(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, Epi epi,
                           float *C, _Float16 *C16, _Float16 *C16lo, int ldc, const float *bias,
                           hipStream_t st) {
-  // Short launches (single requests): 32 x 32 tiles over two LDS stages when fewer than 128 tiles of
-  // 64 x 64 cover the output, else 64 x 128 tiles when fewer than 256 of 128 x 128 would; the same
-  // per-element sequence, so the same bits (a 144-token request on the 24-layer d2048 model 8.46 ->
-  // 4.97 ms, 560 tokens 9.66 -> 8.29 ms, 1024 tokens 11.89 -> 10.35 ms).
+  // Calls come here as launch_kind says.  Short launches: 32 x 32 tiles over two LDS stages when fewer than 128
+  // tiles of 64 x 64 cover the output, else 64 x 128 tiles when fewer than 256 of 128 x 128 would; the same
+  // per-element sequence, so the same bits.
   if (W.cols % 128 == 0) {
     const bool glu = epi == Epi::SWIGLU || epi == Epi::GEGLU;
     const int outN = glu ? W.rows / 2 : W.rows;
@@ -39,7 +38,7 @@ bool launch_gemm_q4_exact(const _Float16 *A, const _Float16 *Alo, int M, const D
   // the Q8_0 geometry: 128 x 128 x 64 tiles, one LDS stage (the correction's four planes size it)
   LG_REQUIRE(ks, "gemm: an exact Q4_K launch needs its activation's chunk sums");
   // short launches: 32 x 128 tiles over two LDS stages, or 64 x 128 tiles (the Q8_0 rule with the
-  // 128 x 128 tiles kept from 192 of them: at 224, a 1024-token request's o projection, they are faster)
+  // 128 x 128 tiles kept from 192 of them: at 224 they are faster)
   if (W.cols % 128 == 0) {
     const bool glu = epi == Epi::SWIGLU || epi == Epi::GEGLU;
     const int outN = glu ? W.rows / 2 : W.rows;
