@@ -919,9 +919,9 @@ void Engine::run_layers_prefill(BatchPlan &b, lg_cancel_fn cancel, void *arg) {
   // them (10 us and 8 bytes a value at 4.3 TB/s).  The rows' way wins where the rotating epilogue has only 64-column tiles:
   // head_dim 64 at thousands of rows (F16 2048 x 3072: 2,500 rows 92 us fused against 85, 8,192 314 / 238, 32,768 1211 / 842),
   // and head_dim 128 just below the 256 x 256 tiles (F16 4608 x 3584: 1,640 rows 179 / 152).  The pass takes up to 40 us more
-  // where a request's length is no multiple of four (16 KV heads of 128: 1,100 rows 109 us fused, 131-144 by rows), hence
+  // where a request's length is no multiple of four (16 KV heads of 128: 1,251 rows 102 us fused, 125 by rows), hence
   // the margin at head_dim 128.
-  const float margin = hd == 64 ? 1.1f : 1.25f;
+  const float margin = hd == 64 ? 1.1f : 1.28f;
   std::vector<uint8_t> fused(L, 0);
   for (int l = 0; l < L && split(); ++l) {
     const std::vector<ProjPart> &parts = layers_[l].qkv;

@@ -58,8 +58,8 @@ __global__ __launch_bounds__(kT) void rmsnorm_kernel(const float *__restrict__ x
 
 // The same into f16 (+ lo plane) for d % 4 == 0, d <= 1024 NI: the row and the weights are loaded together, as float4 at
 // clamped indices (no load waits for the sum of squares or for another), and kept in registers; one barrier.  Latency-bound for
-// a request's rows (weights after the sum, a shuffle reduction and two barriers: 3.3 us against 2.7 for 144 rows of 512),
-// HBM-bound for a batch's (34,560 rows of 2048: 91.3 -> 87.1 us).
+// a request's rows (weights after the sum, a shuffle reduction and two barriers: 3.3 us against 2.8 for 144 rows of 512),
+// HBM-bound for a batch's (34,560 rows of 2048: 91.3 -> 89.2 us).
 template <int NI>
 __global__ __launch_bounds__(kT) void rmsnorm_f16_vec_kernel(const float *__restrict__ x, int d,
                                                              const float *__restrict__ w, float eps,

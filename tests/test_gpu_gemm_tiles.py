@@ -75,11 +75,11 @@ def test_long_vocabulary_argmax(lh):
 
 
 @pytest.mark.parametrize("preset, layers, counts", [
-    ("f16-7b", 1, (4 * (528,), 8 * (512,), 8 * (672,))), ("q8-2048", 1, (4 * (410,), 7 * (401, 431))),
+    ("f16-7b", 1, (4 * (528,), 8 * (512,), 8 * (672,), 2 * (1640,))), ("q8-2048", 1, (4 * (410,), 7 * (401, 431), 2 * (1600,))),
     ("q4km-7b", 1, (10 * (440,) + 3 * (131,),)), ("laya-english", 1, (13 * (479,) + 21 * (45,),))])
 def test_qkv_rule_rows(lh, preset, layers, counts):
-    """Row counts where the rotating q|k|v launch goes from the 64-column tiles to the 256 x 256 ones: a request's bits do
-    not change with the launch that its batch takes."""
+    """Row counts where the rotating q|k|v launch goes from the 64-column tiles to the 256 x 256 ones, or to f32 rows and a RoPE
+    pass (1,640 F16 rows alone): a request's bits do not change with the launch that its batch takes."""
     eng = lh.Engine(lh.Gguf.from_bytes(lh.SynthImage(preset, seed=31, n_layers=layers)), kv_tokens=16384)
     rng = np.random.default_rng(11)
 
