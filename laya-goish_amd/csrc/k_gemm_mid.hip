@@ -188,12 +188,15 @@ float long_cost(int M, const DevMatrix &W, bool glu, bool rope) {
   return t == kNoTile ? INFINITY : c * kLong[mode][t];
 }
 
-// The 256 x 256 tiles (where they take the launch) or those of gemm_mid.h (where they do); *us, if asked for: the modelled microseconds.  Fewer 256 x 256 tiles than 5/8 of the CUs leaves too many idle.  Between that and one tile per CU they still win (F16 at 1437 rows x 7168 gated, 168 tiles: 47.8 us against 53.4 of the best smaller tiles), and below it they lose.  A last round that is nearly empty
-// loses too (301 rows x 37888 gated F16, 296 tiles, against 170 us), so up to two rounds the modelled costs decide, with 8%
-// for the larger tiles: over 60 shapes and row counts the choice is the faster one or within 4% of it (F16 3584 x 18944 at
-// 3,000 rows 757 us against 892, at 4,800 rows 1623 against 1529; Q4_K 3584 x 3584 at 4,800 rows 371 against 432).  Over more
-// the card holds its power and the larger tiles, with fewer instructions an MFMA, win whatever their last round (the
-// 16-request Q4_K/Q6_K batch, 3.5 rounds of Q6_K down: 31.4 against 34.0 ms).
+// The 256 x 256 tiles (where they take the launch) or those of gemm_mid.h (where they do); *us, if asked for: the
+// modelled microseconds.  Fewer 256 x 256 tiles than 5/8 of the CUs leaves too many idle.  Between that and one tile
+// per CU they still win (F16 at 1437 rows x 7168 gated, 168 tiles: 47.8 us against 53.4 of the best smaller tiles), and
+// below it they lose.  A last round that is nearly empty loses too (301 rows x 37888 gated F16, 296 tiles, against 170
+// us), so up to two rounds the modelled costs decide, with 8% for the larger tiles: over 60 shapes and row counts the
+// choice is the faster one or within 4% of it (F16 3584 x 18944 at 3,000 rows 757 us against 892, at 4,800 rows 1623
+// against 1529; Q4_K 3584 x 3584 at 4,800 rows 371 against 432).  Over more the card holds its power and the larger
+// tiles, with fewer instructions an MFMA, win whatever their last round (the 16-request Q4_K/Q6_K batch, 3.5 rounds of
+// Q6_K down: 31.4 against 34.0 ms).
 GemmForm choose(int M, const DevMatrix &W, bool wide_takes, bool mid_takes, bool glu, bool rope, float *us) {
   const int64_t n = device_cus(), tiles = int64_t((M + wide::BM - 1) / wide::BM) * (W.rows / wide::BN);
   const auto mid_us = [&] { return mid_takes ? long_cost(M, W, glu, rope) : INFINITY; };
