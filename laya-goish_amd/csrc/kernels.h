@@ -196,8 +196,9 @@ enum class GemmForm { None, Mid, Wide };
 GemmForm gemm_form(int M, const DevMatrix &W, Epi epi, float *us = nullptr);
 GemmForm gemm_rope_form(int M, const DevMatrix &W, int hd, float *us = nullptr);  // q|k|v of a decoder, rotating epilogue
 GemmForm gemm_laya_rope_form(int M, const DevMatrix &W, int heads);               // q|k|v of an encoder, rotating epilogue
-// The two rotating q|k|v launches above on the tiles of gemm_mid.h, for any M, in the exact split mode: the same bits as the F32 GEMM followed by the RoPE kernel.  head_dim 64 or 128, ro.col0 a
-// multiple of it; anything the takes function refuses fails.  The encoder's needs F16 weights.
+// The two rotating q|k|v launches above on the tiles of gemm_mid.h, for any M, in the exact split mode: the same
+// bits as the F32 GEMM followed by the RoPE kernel.  head_dim 64 or 128, ro.col0 a multiple of it; anything the
+// takes function refuses fails.  The encoder's needs F16 weights.
 bool gemm_mid_rope_takes(int M, const DevMatrix &W, int hd);
 void launch_gemm_mid_rope(const _Float16 *A, const _Float16 *Alo, int M, const DevMatrix &W, const float *bias,
                           const RopeKvOut &ro, hipStream_t st, const _Float16 *ks = nullptr);
